@@ -181,7 +181,11 @@ __device__ __forceinline__ void load_codebook_lds(uint8_t* lds, const uint8_t* t
 }
 __device__ __forceinline__ void load_codebook_lds(uint8_t* lds) { load_codebook_lds(lds, g_codebook_e4m3); }
 template <int THREADS>
-__device__ __forceinline__ void load_codebook_lds_t(uint8_t* lds) { copy_table_lds<65536, THREADS>(lds, g_codebook_e4m3); }
+__device__ __forceinline__ void load_codebook_lds_t(uint8_t* lds, const uint8_t* table) {
+  copy_table_lds<65536, THREADS>(lds, table);
+}
+template <int THREADS>
+__device__ __forceinline__ void load_codebook_lds_t(uint8_t* lds) { load_codebook_lds_t<THREADS>(lds, g_codebook_e4m3); }
 template <int THREADS>
 __device__ __forceinline__ void load_codebook16_lds(uint8_t* lds) {
   copy_table_lds<131072, THREADS>(lds, g_codebook_f16);

@@ -88,3 +88,41 @@ def test_joined_from_expert_layer(cuda, orc):
     err = rel_l2(got, bits_to_f32(want))
     say(f"rel L2 {err:.2e}")
     assert err <= 1e-3
+
+
+@pytest.mark.parametrize("kind", ["plain", "signs", "zero unit", "any unit", "beyond fp16"])
+@pytest.mark.parametrize("k,n,side", [(128, 128, 2), (384, 256, 1), (512, 128, 1), (1024, 256, 2), (640, 128, 2)])
+def test_encode_projection_edges(cuda, orc, k, n, side, kind):
+    """One projection with ragged input steps (K % 256, K % 512), both storage orders and every form
+    of the side vectors: none, +-1 signs, zeros, products that are not fp16 numbers, and products
+    beyond the fp16 range.  Rows outside the projection's stay as they were."""
+    from mlxlr8_amd._lib import check, lib, ptr, stream
+    say(f"encode projection {k} x {n}, side {side}, {kind}")
+    rng = np.random.default_rng(7 * k + n + side)
+    experts, rows, offset = 3, n + 160, 32
+    packed = rng.integers(0, 256, experts * k * n // 2, np.uint8)
+    scale = unit = None
+    if kind != "plain":
+        scale = np.exp(rng.normal(-3, 2, (experts, k))).astype(np.float16) * rng.choice([-1, 1], (experts, k)).astype(np.float16)
+        unit = rng.choice([-1, 1], k).astype(np.float16)
+        if kind == "zero unit":
+            unit[rng.integers(0, k, 20)] = 0
+            unit[64:96] = 0
+        elif kind == "any unit":
+            unit[: k // 2] = rng.normal(0, 0.3, k // 2).astype(np.float16)
+            scale[1] = (rng.integers(1, 40, k) * 2.0 ** -24).astype(np.float16)
+        elif kind == "beyond fp16":
+            scale[:, ::7] = 60000
+            unit[::14] = 3
+    want = (np.full((experts, rows, k // 2), 0xA5, np.uint8), np.full((experts, rows, k // 32), 0x5A, np.uint8))
+    bits = [None if v is None else v.view(np.uint16) for v in (scale, unit)]
+    got = [torch.from_numpy(w.copy()).to(cuda) for w in want]
+    orc.k4_to_mxfp4(packed, k, n, side, experts, *bits, *want, offset)
+    pk = torch.from_numpy(packed).to(cuda)
+    sv = [None if v is None else torch.from_numpy(v).to(cuda) for v in (scale, unit)]
+    ws = torch.empty(lib().moe_k4_to_mxfp4_workspace_bytes(k, n), dtype=torch.uint8, device=cuda)
+    check(lib().moe_k4_to_mxfp4(ptr(pk), pk.numel(), k, n, side, *(None if v is None else ptr(v) for v in sv),
+                                ptr(got[0]), ptr(got[1]), rows, offset, ptr(ws), ws.numel(), stream(cuda)))
+    torch.cuda.synchronize()
+    for name, g, w in zip(("codes", "scales"), got, want):
+        np.testing.assert_array_equal(g.cpu().numpy(), w, err_msg=name)
