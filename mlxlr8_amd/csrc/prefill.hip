@@ -26,12 +26,19 @@
 //     nibble j (low nibble first) is k = 32(l/16)+j; lane l's scale byte scales k-block l/16.  The
 //     fp16 MFMAs of a 128-wide k step reuse the lane's 32 widened weights: MFMA q (q = 0..3) maps
 //     its k-group kg = l/16 to k = 32 kg + 8q + i, and the staged hi activations are read to match.
-//   * A work item is (block of <= 64 sorted rows of one expert, output block): the weights of the
-//     output block are streamed once per item with 16 B loads per lane; the item's activation
-//     terms for one 128-wide k step are staged in LDS (double buffered) and shared by the 8 waves.
-//   * The gate finish (both 128-column halves of an intermediate block are in one item) and the
-//     down finish (H128 over the item's 128 output columns) run in the GEMM epilogues through LDS;
-//     the gate epilogue writes the down GEMM's fp8 terms directly.
+//   * A unit of work is (plan block of <= 64 sorted rows of one expert, 512 weight rows): one
+//     persistent 8-wave block per CU claims units, and the loads of the next unit are in flight while
+//     the one before is finished.  The unit's activation records of one or two 128-wide k steps are
+//     staged in LDS (double buffered) and shared by the 8 waves, each of which streams the 64 weight
+//     rows of its four column tiles with 16 B loads per lane.
+//   * The gate finish (a pass holds the gate and up rows of the same intermediate columns) and the
+//     down finish (H128 over 128 output columns) run per unit through LDS; the gate finish writes the
+//     down GEMM's records directly.
+//   * Measured (GLM-5.3 layer, whole routed block, the start of each row being one item per workgroup
+//     of 64 rows x 256 columns or 32 x 512, padded rows in LDS and a byte store per term):
+//     24 rows 742 -> 618 us, 512 rows 1,596 -> 1,350 us, 2,048 rows 4,730 -> 3,154 us, same outputs.
+//     What bounds it: 24 rows, the weight stream (2.8 GB at 4.7 TB/s; the same loads alone reach 5.8);
+//     2,048 rows, the matrix cores (busy 53% of the cycles) and 14 GB of activation and weight reads.
 #include <hip/hip_runtime.h>
 
 #include "moe_device.h"
@@ -42,6 +49,7 @@ namespace {
 
 typedef int i32x8 __attribute__((ext_vector_type(8)));
 typedef int i32x4 __attribute__((ext_vector_type(4)));
+typedef int i32x2 __attribute__((ext_vector_type(2)));
 
 __device__ __forceinline__ f16x8 pack_f16x8(f16x2 a, f16x2 b, f16x2 c, f16x2 d) {
   typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
@@ -52,19 +60,14 @@ __device__ __forceinline__ f16x8 pack_f16x8(f16x2 a, f16x2 b, f16x2 c, f16x2 d) 
 constexpr int kPfItemRows = 64;  // sorted rows per GEMM work item (4 M-tiles of 16)
 constexpr int kPfWaves = 8;      // waves per GEMM block
 constexpr int kPfThreads = kPfWaves * 64;
-constexpr int kPfRowBytes = 528; // LDS row stride of a staged k step: 256 B hi + 2 x 128 B lo + pad
+constexpr int kPfTiles = 4;      // 16-column tiles per wave
+constexpr int kPfCols = kPfWaves * kPfTiles * 16;  // weight rows (output columns) per pass of an item
+constexpr int kPfRecord = 512;   // bytes of a row's 128-wide k step: 256 hi + 2 x 128 remainder codes
 constexpr int kPfLo = 2;         // fp8 remainder terms
 constexpr int kPfMaxExperts = 1024;
-constexpr size_t kPfMaxLds = 160 * 1024;  // LDS per workgroup on gfx950
-#ifndef MOE_PF_MERGE_GATE
-#define MOE_PF_MERGE_GATE 1
-#endif
-#ifndef MOE_PF_DOWN_TWO
-#define MOE_PF_DOWN_TWO 1
-#endif
-#ifndef MOE_PF_MERGE_DOWN
-#define MOE_PF_MERGE_DOWN 0
-#endif
+constexpr int kPfQueueLine = 32;                                // words between claim counters (128 B)
+constexpr int kPfQueueWords = 2 * 4 * 8 * kPfQueueLine;         // [GEMM][class][XCD]
+constexpr int kPfMaxHidden = 8080, kPfMaxIntermediate = 16160;  // largest sizes the entries take
 
 // ---------------------------------------------------------------- sorted work order
 // One block of 1024 threads (16 waves).  Counting sort of the flat ids (stable: slots of one
@@ -212,12 +215,51 @@ __device__ __forceinline__ uint32_t hi_lo_terms(float v0, float v1, uint32_t (&l
   return (uint32_t)__builtin_bit_cast(uint16_t, h0) | ((uint32_t)__builtin_bit_cast(uint16_t, h1) << 16);
 }
 
+// A row's 128 values of one k step as a record of kPfRecord bytes in the MFMAs' operand order: for
+// each k-group g = 0..3 (lanes 16 g .. 16 g + 15 of the matrix instructions) 64 B of hi (k = 32 g ..
+// 32 g + 31 as fp16) and per remainder term 32 B of codes (k = 16 g + j, then k = 64 + 16 g + j).
+// Called by one wave, whose lane l holds the values 2 l and 2 l + 1.
+__device__ __forceinline__ void store_record(uint8_t* rec, uint32_t hi, const uint32_t (&lo)[kPfLo]) {
+  const int lane = lane_id();
+  *reinterpret_cast<uint32_t*>(rec + lane / 16 * 128 + lane % 16 * 4) = hi;
+#pragma unroll
+  for (int t = 0; t < kPfLo; t++)
+    *reinterpret_cast<uint16_t*>(rec + lane % 32 / 8 * 128 + 64 + 32 * t + lane / 32 * 16 + lane % 8 * 2) = (uint16_t)lo[t];
+}
+
 // xh = H128(x * unit) of every token -> hi/lo terms.  One wave per (token, 128-block).
-// xh_hi: [rows][K] fp16, xq: [kPfLo][rows][K] fp8 remainder terms, xs: [kPfLo][rows][K/32] e8m0.
+// xa: [rows][K/128] records, xs: [kPfLo][rows][K/32] e8m0.
+// The last block of the grid prepares the GEMMs' work lists instead (it needs only the segment table,
+// which ran before): ent lists the plan blocks by M-tiles, most first, ends[c] is the end of the blocks
+// of 4 - c M-tiles in it, and the claim counters are cleared.
 __global__ __launch_bounds__(256) void prep_terms_kernel(const uint16_t* __restrict__ x,
                                                          const uint16_t* __restrict__ unit, int rows, int K,
-                                                         uint16_t* __restrict__ xh_hi, uint8_t* __restrict__ xq,
-                                                         uint8_t* __restrict__ xs) {
+                                                         uint8_t* __restrict__ xa, uint8_t* __restrict__ xs,
+                                                         const int32_t* __restrict__ blk,
+                                                         int cap, const int32_t* __restrict__ nblk,
+                                                         int32_t* __restrict__ ent, int32_t* __restrict__ ends,
+                                                         int32_t* __restrict__ queue) {
+  if (blockIdx.x == gridDim.x - 1) {
+    __shared__ int32_t cnt[5], pos[5];
+    if (threadIdx.x < 5) cnt[threadIdx.x] = 0;
+    for (int i = threadIdx.x; i < kPfQueueWords; i += 256) queue[i] = 0;
+    __syncthreads();
+    const int nb = min(*nblk, cap);
+    auto tiles = [&](int b) { return min(max((blk[2 * cap + b] + 15) / 16, 1), 4); };
+    for (int b = threadIdx.x; b < nb; b += 256) atomicAdd(&cnt[tiles(b)], 1);
+    __syncthreads();
+    if (threadIdx.x == 0) {
+      int run = 0;
+      for (int t = 4; t >= 1; t--) {
+        pos[t] = run;
+        run += cnt[t];
+        ends[4 - t] = run;
+      }
+    }
+    __syncthreads();
+    for (int b = threadIdx.x; b < nb; b += 256) ent[atomicAdd(&pos[tiles(b)], 1)] = b;
+    return;
+  }
   const int64_t wid = (int64_t)blockIdx.x * 4 + wave_id_uniform();
   const int blocks = K / 128;
   if (wid >= (int64_t)rows * blocks) return;
@@ -231,12 +273,10 @@ __global__ __launch_bounds__(256) void prep_terms_kernel(const uint16_t* __restr
   hadamard128_wave(v0, v1);
   uint32_t lo[kPfLo], sc[kPfLo];
   const uint32_t hi = hi_lo_terms(v0, v1, lo, sc);
-  *reinterpret_cast<uint32_t*>(xh_hi + (int64_t)t * K + k0) = hi;
+  store_record(xa + wid * kPfRecord, hi, lo);
 #pragma unroll
-  for (int tt = 0; tt < kPfLo; tt++) {
-    *reinterpret_cast<uint16_t*>(xq + ((int64_t)tt * rows + t) * K + k0) = (uint16_t)lo[tt];
+  for (int tt = 0; tt < kPfLo; tt++)
     if ((lane & 15) == 0) xs[((int64_t)tt * rows + t) * (K / 32) + b * 4 + lane / 16] = (uint8_t)sc[tt];
-  }
 }
 
 // ---------------------------------------------------------------- grouped GEMM machinery
@@ -245,11 +285,8 @@ struct PfGemm {
   const uint8_t* codes;
   const uint8_t* wscales;
   int K, N;
-  // activation terms: ahi [arows][K] fp16, aq [kPfLo][arows][K] fp8 remainder terms,
-  // as [kPfLo][arows][K/32] e8m0;
-  // the row of sorted position p is rowmap ? rowmap[p] / rowdiv : p
-  const uint16_t* ahi;
-  const uint8_t* aq;
+  // activation terms: aa [arows][K/128] records, as [kPfLo][arows][K/32] e8m0; the row of sorted position p is rowmap ? rowmap[p] / rowdiv : p
+  const uint8_t* aa;
   const uint8_t* as;
   int64_t arows;
   const int32_t* rowmap;
@@ -257,15 +294,16 @@ struct PfGemm {
   // plan
   const int32_t* blk;  // [3][cap]
   int cap;
-  const int32_t* nblk;
+  const int32_t* ent;    // plan blocks in launch order (most M-tiles first)
+  const int32_t* ends;   // end of the blocks of 4, 3, 2, 1 M-tiles in ent
+  int32_t* queue;        // claim counters [class][XCD], one line each
   const int32_t* order;  // sorted position -> slot
-  // gate epilogue (N = 2m): hidden terms hhi [n][m] fp16, hq [kPfLo][n][m] fp8, hs [kPfLo][n][m/32]
+  // gate epilogue (N = 2m): hidden terms ha [n][m/128] records, hs [kPfLo][n][m/32]
   const uint16_t* out_gate;
   const uint16_t* out_up;
   const uint16_t* in_down;
   int m;
-  uint16_t* hhi;
-  uint8_t* hq;
+  uint8_t* ha;
   uint8_t* hs;
   int64_t nslots;
   // down epilogue: values [slots][N] bf16
@@ -273,419 +311,537 @@ struct PfGemm {
   uint16_t* values;
 };
 
-// Staging of one 128-wide k step of the item's activations: per row [256 B hi][128 B lo1][128 B lo2]
-// at stride kPfRowBytes, and the row's 4 scales of each remainder term.
+// Shape of the items of MT M-tiles (16 rows each).
+//   kSteps    128-wide k steps per activation stage (one block barrier per stage)
+//   kRing     k steps of weights in flight per wave
+//   kBurst    k steps of a weight row loaded back to back: two 64 B halves make one request of whole
+//             lines (streaming 16 rows this way reaches 5.8 TB/s, one half at a time 4.9)
+//   kScSteps  k steps of weight scales per LDS chunk
+//   kAhead    MFMA groups (64 cycles each) whose LDS reads are in flight
+// Items of one or two M-tiles are bound by the weight stream, items of three or four by the matrix
+// cores: there two steps in flight keep accumulators, weights and the next stage within 256 VGPRs.
 template <int MT>
-struct PfStage {
-  static constexpr int kBytes = MT * 16 * kPfRowBytes;
-  static constexpr int kScaleBytes = MT * 16 * 4 * kPfLo;
+struct PfShape {
+  static constexpr int kSteps = MT <= 2 ? 2 : 1;
+  static constexpr int kRing = MT <= 2 ? 4 : 2;
+  static constexpr int kBurst = MT <= 2 ? 2 : 1;
+  static constexpr int kScSteps = 16;
+  static constexpr int kAhead = MT == 1 ? 4 : MT == 2 ? 3 : 2;
+  static constexpr int kRows = MT * 16;
+  static constexpr int kStepBytes = kRows * kPfRecord;                  // one k step's rows
+  static constexpr int kStageBytes = kSteps * kStepBytes;               // per buffer (two of them)
+  static constexpr int kAScales = kSteps * kRows * kPfLo;               // scale dwords per stage
+  static constexpr int kScRow = kScSteps * 4 + 8;                       // LDS row of scales (padded: no bank conflicts)
+  static constexpr int kScBytes = kPfTiles * 16 * kScRow;               // weight scales per wave
+  static constexpr int kChunks = kSteps * kRows * 32 / kPfThreads;      // 16 B chunks per thread and stage
 };
 
-// A k step's activation chunks in flight in registers: thread t holds chunks t + kPfThreads i
-// (16 B each; MT * 16 rows x 32 chunks = MT chunks per thread) and at most one scale dword.
+// LDS: the finish's exchange (one M-tile), two activation stages, their scales, the row map, the claimed
+// unit, per wave a chunk of weight scales.  One block per CU: its 512 columns halve the activation
+// traffic of two blocks of 256 (which was 14 of 23 GB at 2048 rows).
+constexpr int kPfExchange = 16 * kPfCols * 4;
+template <int MT>
+__host__ __device__ constexpr int pf_shape_lds() {
+  return kPfExchange + 2 * PfShape<MT>::kStageBytes + 2 * PfShape<MT>::kAScales * 4 + PfShape<MT>::kRows * 8 + 16 +
+         kPfWaves * PfShape<MT>::kScBytes;
+}
+constexpr int kPfLds = pf_shape_lds<4>() > pf_shape_lds<2>() ? pf_shape_lds<4>() : pf_shape_lds<2>();
+static_assert(pf_shape_lds<1>() <= kPfLds && pf_shape_lds<3>() <= kPfLds, "the largest shapes set the LDS size");
+static_assert(kPfLds <= 160 * 1024, "LDS of a CU");
+
+// A stage's activation chunks in flight in registers: thread t holds the 16 B chunks t + kPfThreads i
+// (row and step i * kPfThreads / 32 + t / 32, chunk t % 32 of the record) and at most one scale dword.
 template <int MT>
 struct PfFetch {
-  i32x4 v[MT];
+  i32x4 v[PfShape<MT>::kChunks];
   uint32_t sc;
 };
-// Where a thread's chunks come from: chunk i is row r = t / 32 + 16 i of the item (t = thread) and
-// chunk t % 32 of the row (0-15: hi, 16-23: lo1, 24-31: lo2); the addresses are fixed per item up
-// to the k step offset, so they are formed once per item.
+// Where a thread's chunks come from and go to.
 template <int MT>
 struct PfSrc {
-  const uint8_t* p[MT];  // chunk i at k step 0
-  const uint8_t* sp;     // the thread's scale dword at k step 0
-  int step;              // bytes per k step of the thread's chunks: 256 (hi) or 128 (lo)
+  static constexpr int kRowsPer = PfShape<MT>::kChunks / PfShape<MT>::kSteps;  // chunks per k step
+  const uint8_t* base;     // the thread's chunk of row 0 at k step 0
+  uint32_t row[kRowsPer];  // the i-th row's first record
+  const uint8_t* sp;       // the thread's scale dword at stage 0
 };
 template <int MT>
 __device__ __forceinline__ void item_src(const PfGemm& a, const int64_t* rowidx, PfSrc<MT>& s) {
-  constexpr int kPer = 16 + 8 * kPfLo;
-  static_assert(MT * 16 * kPer == MT * kPfThreads, "one chunk per thread and M-tile");
-  const int ch = (int)threadIdx.x % kPer;
-  s.step = ch < 16 ? 256 : 128;
+  using S = PfShape<MT>;
+  s.base = a.aa + threadIdx.x % 32 * 16;
 #pragma unroll
-  for (int i = 0; i < MT; i++) {
-    const int r = (int)threadIdx.x / kPer + i * (kPfThreads / kPer);
-    if (ch < 16) {
-      s.p[i] = reinterpret_cast<const uint8_t*>(a.ahi + rowidx[r] * a.K) + ch * 16;
-    } else {
-      const int t = (ch - 16) / 8, cc = (ch - 16) % 8;
-      s.p[i] = a.aq + (t * a.arows + rowidx[r]) * a.K + cc * 16;
-    }
-  }
-  const int c = min((int)threadIdx.x, MT * 16 * kPfLo - 1);
-  const int r = c / kPfLo, t = c % kPfLo;
-  s.sp = a.as + (t * a.arows + rowidx[r]) * (a.K / 32);
+  for (int i = 0; i < PfSrc<MT>::kRowsPer; i++)
+    s.row[i] = (uint32_t)(rowidx[(int)threadIdx.x / 32 + i * (kPfThreads / 32)] * (a.K / 128));
+  const int c = min((int)threadIdx.x, S::kAScales - 1);
+  const int gk = c / (S::kRows * kPfLo), r = c % (S::kRows * kPfLo) / kPfLo, t = c % kPfLo;
+  s.sp = a.as + (t * a.arows + rowidx[r]) * (a.K / 32) + gk * 4;
 }
+// ks: the stage's first k step (a multiple of kSteps; K / 128 is even, so a stage is whole)
 template <int MT>
 __device__ __forceinline__ void fetch_k(const PfSrc<MT>& s, int ks, PfFetch<MT>& f) {
-  const int off = ks * s.step;
+  constexpr int kPer = PfSrc<MT>::kRowsPer;
 #pragma unroll
-  for (int i = 0; i < MT; i++) f.v[i] = *reinterpret_cast<const i32x4*>(s.p[i] + off);
+  for (int i = 0; i < PfShape<MT>::kChunks; i++)
+    f.v[i] = *reinterpret_cast<const i32x4*>(s.base + (ks + i / kPer) * kPfRecord + (uint64_t)s.row[i % kPer] * kPfRecord);
   f.sc = *reinterpret_cast<const uint32_t*>(s.sp + ks * 4);
 }
+// Chunk c = 8 g + h of row r (of 16 in an M-tile) goes to the tile's line c of 256 B, 16 B column
+// r ^ h.  A matrix operand read (lane (nn, g) reads chunk 8 g + h of row nn, one h per instruction)
+// then touches every column once per 16 rows whatever lanes share a cycle, and so do eight
+// neighbouring lanes of these writes: neither has bank conflicts.  (Row-major rows padded to 528 B:
+// 42% of the LDS cycles were conflicts.)
 template <int MT>
 __device__ __forceinline__ void put_k(const PfFetch<MT>& f, uint8_t* buf, uint8_t* sbuf) {
-  constexpr int kPer = 16 + 8 * kPfLo;
+  const int c = (int)threadIdx.x % 32, r0 = (int)threadIdx.x / 32;
+  static_assert(kPfThreads / 32 == 16, "an M-tile's rows per chunk");
+  const uint32_t at = c * 256 + ((r0 ^ (c & 7)) * 16);
 #pragma unroll
-  for (int i = 0; i < MT; i++) {
-    const int c = threadIdx.x + i * kPfThreads;
-    *reinterpret_cast<i32x4*>(buf + (c / kPer) * kPfRowBytes + (c % kPer) * 16) = f.v[i];
-  }
-  if ((int)threadIdx.x < MT * 16 * kPfLo) *reinterpret_cast<uint32_t*>(sbuf + threadIdx.x * 4) = f.sc;
+  for (int i = 0; i < PfShape<MT>::kChunks; i++)
+    *reinterpret_cast<i32x4*>(buf + at + i * 16 * kPfRecord) = f.v[i];
+  // threads past the scales hold (and write) the last one again
+  *reinterpret_cast<uint32_t*>(sbuf + min((int)threadIdx.x, PfShape<MT>::kAScales - 1) * 4) = f.sc;
 }
 
-// The item's rows: sorted positions [first, first + len), clamped into the item for the padding
-// rows of the last M-tile (their results are discarded).
+// A lane's place in a staged k step: chunk h of row nn and k-group g of an M-tile, and the row's scales.
+// Opaque to the compiler, so that every LDS read of the loop is one of these registers plus an
+// immediate offset (it otherwise keeps an address per M-tile and stage, and spills).
+struct PfLane {
+  uint32_t h[8], sc;
+  __device__ __forceinline__ PfLane() {
+    const int lane = lane_id(), nn = lane & 15, g = lane >> 4;
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+      h[i] = (8 * g + i) * 256 + (nn ^ i) * 16;
+      asm volatile("" : "+v"(h[i]));
+    }
+    sc = nn * kPfLo * 4;
+    asm volatile("" : "+v"(sc));
+  }
+};
+
+// The two MFMA phases of a k step.  ab = the staged rows, sb = their scales [row][term][4], (bw, bs) =
+// the weights.  Each group of MFMAs is issued after the LDS reads of the next group (the scheduling
+// fences keep that order; without them every group waits for its own reads and the matrix cores run
+// at half rate).
+//
+// hi: 4 fp16 MFMAs per M-tile and column tile; the q-th reads k = 32 g + 8 q + i, i.e. the 8 codes of
+// word q, widened to fp16 with their block scale one q ahead of their use.
+__device__ __forceinline__ f16x8 widen(uint32_t word, float scale) {
+  return pack_f16x8(
+      __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(word, scale, 0), __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(word, scale, 1),
+      __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(word, scale, 2), __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(word, scale, 3));
+}
+struct PfLoRows {
+  i32x4 l0, l1;
+};
+// remainder rows of group i = (M-tile i / kPfLo, term i % kPfLo)
+__device__ __forceinline__ PfLoRows lo_rows(const uint8_t* ab, const PfLane& at, int i) {
+  const uint8_t* p = ab + i / kPfLo * 16 * kPfRecord;
+  const int t = i % kPfLo;
+  return PfLoRows{*reinterpret_cast<const i32x4*>(p + at.h[4 + 2 * t]), *reinterpret_cast<const i32x4*>(p + at.h[5 + 2 * t])};
+}
+// lo and asc: the first remainder rows and the scales, for gemm_lo
 template <int MT>
-__device__ __forceinline__ void item_rows(const PfGemm& a, int first, int len, int64_t* rowidx) {
+__device__ __forceinline__ void gemm_hi(const uint8_t* ab, const uint8_t* sb, const PfLane& at,
+                                        const i32x4 (&bw)[kPfTiles], const uint32_t (&bs)[kPfTiles],
+                                        f32x4 (&acc)[MT][kPfTiles], PfLoRows& lo, u32x2 (&asc)[MT]) {
+  constexpr int NT = kPfTiles, P = PfShape<MT>::kAhead;  // groups read ahead
+  auto rows = [&](int i) { return *reinterpret_cast<const f16x8*>(ab + at.h[i / MT] + i % MT * 16 * kPfRecord); };
+  f16x8 a[4 * MT];
+#pragma unroll
+  for (int i = 0; i < P; i++) a[i] = rows(i);
+  __builtin_amdgcn_sched_barrier(0);
+  float wsc[NT];
+  f16x8 bh[2][NT];
+#pragma unroll
+  for (int j = 0; j < NT; j++) {
+    wsc[j] = __builtin_amdgcn_ldexpf(1.0f, (int)bs[j] - 127);
+    bh[0][j] = widen((uint32_t)bw[j][0], wsc[j]);
+  }
+#pragma unroll
+  for (int i = 0; i < 4 * MT; i++) {
+    const int q = i / MT, mt = i % MT;
+    if (i + P < 4 * MT) a[i + P] = rows(i + P);
+    if (i == 4 * MT - 2) {
+#pragma unroll
+      for (int m = 0; m < MT; m++) asc[m] = *reinterpret_cast<const u32x2*>(sb + at.sc + m * 16 * kPfLo * 4);
+      lo = lo_rows(ab, at, 0);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int j = 0; j < NT; j++) {
+      acc[mt][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[i], bh[q & 1][j], acc[mt][j], 0, 0, 0);
+      if (q < 3 && j * MT / NT == mt) bh[(q + 1) & 1][j] = widen((uint32_t)bw[j][q + 1], wsc[j]);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  }
+}
+// remainder terms: one scaled MX MFMA each on the resident codes
+template <int MT>
+__device__ __forceinline__ void gemm_lo(const uint8_t* ab, const PfLane& at, const i32x4 (&bw)[kPfTiles],
+                                        const uint32_t (&bs)[kPfTiles], f32x4 (&acc)[MT][kPfTiles], PfLoRows a,
+                                        const u32x2 (&asc)[MT]) {
+  const int g = lane_id() >> 4;
+#pragma unroll
+  for (int i = 0; i < kPfLo * MT; i++) {
+    const int mt = i / kPfLo, t = i % kPfLo;
+    PfLoRows next = a;
+    if (i + 1 < kPfLo * MT) next = lo_rows(ab, at, i + 1);
+    __builtin_amdgcn_sched_barrier(0);
+    const i32x8 al = {a.l0.x, a.l0.y, a.l0.z, a.l0.w, a.l1.x, a.l1.y, a.l1.z, a.l1.w};
+    const int as = (int)((asc[mt][t] >> (8 * g)) & 0xFFu);
+#pragma unroll
+    for (int j = 0; j < kPfTiles; j++) {
+      const i32x8 bv = {bw[j].x, bw[j].y, bw[j].z, bw[j].w, 0, 0, 0, 0};
+      acc[mt][j] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(al, bv, acc[mt][j], 0, 4, 0, as, 0, (int)bs[j]);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    a = next;
+  }
+}
+
+// Buffer over expert e's matrix of `bytes` bytes.
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t expert_rsrc(const uint8_t* p, int e, int64_t bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(p) + e * bytes, 0, (int)bytes, 0x00020000);
+}
+
+// ---------------------------------------------------------------- units of work
+// A unit is (plan block, pass of kPfCols weight rows).  A block per CU claims units, class by class
+// (plan blocks of 4, 3, 2, 1 M-tiles), from its XCD's counter of the class: plan block i of a class
+// belongs to XCD i % 8, whose blocks take its passes one after another and so read its activation
+// rows into one L2.  A block whose own XCD has none left takes from the one with most left.  (A fixed
+// deal of the items left 10 to 30% of the CU time idle at the end of a launch.)
+struct PfUnit {
+  int e, first, len, pass;
+};
+
+template <bool GATE>
+__host__ __device__ __forceinline__ int pf_passes(const PfGemm& a) {
+  return GATE ? a.m / 256 : a.N / kPfCols;
+}
+
+struct PfClass {
+  int32_t* queue;  // the class's counters
+  int begin, n;    // its plan blocks in ent
+  int passes;
+  __device__ __forceinline__ int units(int x) const { return (n - x + 7) / 8 * passes; }  // of XCD x
+};
+// First claim of a unit: lane 0 of one wave adds to its XCD's counter.  The result may be past the
+// XCD's units; pf_settle then looks for another XCD.
+__device__ __forceinline__ int pf_claim(const PfClass& c, int x) {
+  return __hip_atomic_fetch_add(c.queue + x * kPfQueueLine, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+// Claimed number v of XCD x -> 8 * (unit of the XCD) + XCD, or -1 when the class has no unit left.
+// Every failed try follows a counter that others moved to its end, so the loop ends.
+__device__ __forceinline__ int pf_settle(const PfClass& c, int x, int v) {
+  while (v >= c.units(x)) {
+    int most = 0, y = -1;
+    for (int k = 0; k < 8; k++) {
+      const int left =
+          c.units(k) - __hip_atomic_load(c.queue + k * kPfQueueLine, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      if (left > most) {
+        most = left;
+        y = k;
+      }
+    }
+    if (y < 0) return -1;
+    x = y;
+    v = pf_claim(c, x);
+  }
+  return v * 8 + x;
+}
+__device__ __forceinline__ PfUnit pf_unit(const PfGemm& a, const PfClass& c, int claimed) {
+  const int x = claimed % 8, v = claimed / 8;
+  const int b = a.ent[c.begin + x + 8 * (v / c.passes)];
+  return PfUnit{a.blk[b], a.blk[a.cap + b], a.blk[2 * a.cap + b], v % c.passes};
+}
+// The unit's rows: sorted positions [first, first + len), clamped into it for the padding rows of the
+// last M-tile (their results are discarded).
+template <int MT>
+__device__ __forceinline__ void unit_rows(const PfGemm& a, const PfUnit& u, int64_t* rowidx) {
   for (int r = threadIdx.x; r < MT * 16; r += kPfThreads) {
-    const int p = first + min(r, len - 1);
+    const int p = u.first + min(r, u.len - 1);
     rowidx[r] = a.rowmap ? (int64_t)(a.rowmap[p] / a.rowdiv) : (int64_t)p;
   }
 }
 
-// One k step of the MFMAs: activations from the staged buffer, weights from (bw, bs).
-template <int MT, int NT>
-__device__ __forceinline__ void gemm_step(const uint8_t* ab, const uint8_t* sb, const i32x4 (&bw)[NT],
-                                          const uint32_t (&bs)[NT], f32x4 (&acc)[MT][NT]) {
-  const int lane = lane_id(), nn = lane & 15, g = lane >> 4;
-  float wsc[NT];
+// ---------------------------------------------------------------- finishes
+// gate/up: a pass is the intermediate columns [256 pass, +256), their gate rows and their up rows (m
+// further on); wave w owns gate and up tile w of both 128-blocks.  Per M-tile: tiles -> LDS
+// [16][gate, up][256] -> per row and 128-block: H128, scale, SwiGLU, in_down, H128 -> hidden terms.
+template <int MT>
+__device__ __forceinline__ void gate_finish(const PfGemm& a, const PfUnit& u, float* ex, const f32x4 (&acc)[MT][kPfTiles]) {
+  const int w = wave_id_uniform(), lane = lane_id(), nn = lane & 15, g = lane >> 4;
+  const int c0 = 2 * u.pass;  // first 128-block
+  float og[2][2], ou[2][2], id[2][2];
 #pragma unroll
-  for (int j = 0; j < NT; j++) wsc[j] = __builtin_amdgcn_ldexpf(1.0f, (int)bs[j] - 127);
-  // hi: 4 fp16 MFMAs per M-tile; the q-th reads k = 32 g + 8 q + i, i.e. the 8 codes of word q,
-  // widened to fp16 with their block scale just before use
+  for (int bb = 0; bb < 2; bb++)
 #pragma unroll
-  for (int q = 0; q < 4; q++) {
-    f16x8 bh[NT];
-#pragma unroll
-    for (int j = 0; j < NT; j++) {
-      const uint32_t word = (uint32_t)bw[j][q];
-      bh[j] = pack_f16x8(__builtin_amdgcn_cvt_scalef32_pk_f16_fp4(word, wsc[j], 0),
-                         __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(word, wsc[j], 1),
-                         __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(word, wsc[j], 2),
-                         __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(word, wsc[j], 3));
+    for (int i = 0; i < 2; i++) {
+      const int64_t si = (int64_t)u.e * a.m + 128 * (c0 + bb) + 2 * lane + i;
+      og[bb][i] = f16_to_f32(a.out_gate[si]);
+      ou[bb][i] = f16_to_f32(a.out_up[si]);
+      id[bb][i] = f16_to_f32(a.in_down[si]);
     }
-#pragma unroll
-    for (int mt = 0; mt < MT; mt++) {
-      const f16x8 ah =
-          *reinterpret_cast<const f16x8*>(ab + (mt * 16 + nn) * kPfRowBytes + (32 * g + 8 * q) * 2);
-#pragma unroll
-      for (int j = 0; j < NT; j++) acc[mt][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah, bh[j], acc[mt][j], 0, 0, 0);
-    }
-  }
 #pragma unroll
   for (int mt = 0; mt < MT; mt++) {
-    const uint8_t* rp = ab + (mt * 16 + nn) * kPfRowBytes;
-    // remainder terms: one scaled MX MFMA each on the resident codes
 #pragma unroll
-    for (int t = 0; t < kPfLo; t++) {
-      const i32x4 l0 = *reinterpret_cast<const i32x4*>(rp + 256 + 128 * t + 16 * g);
-      const i32x4 l1 = *reinterpret_cast<const i32x4*>(rp + 256 + 128 * t + 64 + 16 * g);
-      const i32x8 al = {l0.x, l0.y, l0.z, l0.w, l1.x, l1.y, l1.z, l1.w};
-      const int asc = sb[((mt * 16 + nn) * kPfLo + t) * 4 + g];
+    for (int j = 0; j < kPfTiles; j++)
 #pragma unroll
-      for (int j = 0; j < NT; j++) {
-        const i32x8 bv = {bw[j].x, bw[j].y, bw[j].z, bw[j].w, 0, 0, 0, 0};
-        acc[mt][j] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(al, bv, acc[mt][j], 0, 4, 0, asc, 0,
-                                                                      (int)bs[j]);
-      }
-    }
-  }
-}
-
-// One wave's NT column tiles (cols[j] .. +16) over all K for the item's MT M-tiles.  The weights
-// and the activations are loaded D k steps ahead into rings of D register sets (set s % D holds
-// step s); a step's activations go to LDS (double buffered) in the step before their use, after
-// that step's MFMAs (D even).  The tiles' block scales for all k steps (16 rows x K/32 bytes per
-// tile, one contiguous span in memory) are copied once per item into the wave's LDS region `wsl`
-// with 16 B loads: a byte load per lane and k step from HBM costs about as much as the weights.
-template <int MT, int NT, int MTMAX, int D>
-__device__ __forceinline__ void gemm_item(const PfGemm& a, int e, const int (&cols)[NT], const int64_t* rowidx,
-                                          uint8_t* abuf, uint8_t* sbuf, uint8_t* wsl, f32x4 (&acc)[MT][NT]) {
-  static_assert(D % 2 == 0, "the LDS stage alternates with the step parity");
-  const int lane = lane_id(), nn = lane & 15, g = lane >> 4;
-  const int ksteps = a.K / 128, last = ksteps - 1;
+      for (int i = 0; i < 4; i++)
+        ex[((4 * g + i) * 2 + (j & 1)) * 256 + 128 * (j >> 1) + 16 * w + nn] = acc[mt][j][i];
+    __syncthreads();
+#pragma unroll 1  // one row at a time: registers
+    for (int rr = 0; rr < 2; rr++) {
+      const int r = 2 * w + rr;  // 8 waves x 2 rows
+      const int pr = mt * 16 + r;
+      if (pr < u.len) {
 #pragma unroll
-  for (int mt = 0; mt < MT; mt++)
-#pragma unroll
-    for (int j = 0; j < NT; j++) acc[mt][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-  const int sb = a.K / 32;  // scale bytes per weight row
-#pragma unroll
-  for (int j = 0; j < NT; j++) {
-    const uint8_t* src = a.wscales + ((int64_t)e * a.N + cols[j]) * sb;
-    uint8_t* dst = wsl + j * 16 * sb;
-    for (int c = lane; c < sb; c += 64)  // 16 sb bytes = sb chunks of 16 B
-      *reinterpret_cast<i32x4*>(dst + 16 * c) = *reinterpret_cast<const i32x4*>(src + 16 * c);
-  }
-  const uint8_t* wrow[NT];
-  const uint8_t* srow[NT];
-#pragma unroll
-  for (int j = 0; j < NT; j++) {
-    wrow[j] = a.codes + ((int64_t)e * a.N + cols[j] + nn) * (a.K / 2) + g * 16;
-    srow[j] = wsl + (j * 16 + nn) * sb + g;
-  }
-  constexpr int kStage = PfStage<MTMAX>::kBytes, kSStage = PfStage<MTMAX>::kScaleBytes;
-  auto load_w = [&](i32x4 (&bw)[NT], uint32_t (&bs)[NT], int ks) {
-#pragma unroll
-    for (int j = 0; j < NT; j++) {
-      bw[j] = *reinterpret_cast<const i32x4*>(wrow[j] + ks * 64);
-      bs[j] = srow[j][ks * 4];  // LDS; written above by this wave
-    }
-  };
-  PfSrc<MT> src;
-  item_src<MT>(a, rowidx, src);
-  PfFetch<MT> f[D];
-  i32x4 bw[D][NT];
-  uint32_t bs[D][NT];
-  fetch_k<MT>(src, 0, f[0]);
-  put_k<MT>(f[0], abuf, sbuf);
-#pragma unroll
-  for (int d = 0; d < D; d++) load_w(bw[d], bs[d], min(d, last));
-#pragma unroll
-  for (int d = 1; d <= D; d++) fetch_k<MT>(src, min(d, last), f[d % D]);
-  __syncthreads();
-  for (int ks = 0; ks < ksteps; ks += D) {
-#pragma unroll
-    for (int u = 0; u < D; u++) {
-      const int t = ks + u;  // block-uniform
-      if (t < ksteps) {
-        gemm_step<MT, NT>(abuf + (u & 1) * kStage, sbuf + (u & 1) * kSStage, bw[u], bs[u], acc);
-        load_w(bw[u], bs[u], min(t + D, last));
-        if (t + 1 < ksteps) put_k<MT>(f[(u + 1) % D], abuf + ((u + 1) & 1) * kStage, sbuf + ((u + 1) & 1) * kSStage);
-        fetch_k<MT>(src, min(t + 1 + D, last), f[(u + 1) % D]);
-        __syncthreads();
-      }
-    }
-  }
-}
-
-// ---------------------------------------------------------------- gate/up GEMM + gate finish
-// Item = (plan block b, intermediate blocks c NB .. c NB + NB - 1 of 128): for each block cb the
-// gate columns [128 cb, +128) and the up columns [m + 128 cb, +128); wave w owns gate and up tile
-// 16w of each block (tiles 2 bb, 2 bb + 1).  More blocks per item share each staged activation step
-// among more weights.
-template <int MT, int MTMAX, int NB>
-__device__ __forceinline__ void gateup_item(const PfGemm& a, int e, int first, int len, int c, uint8_t* abuf, uint8_t* sbuf,
-                                            uint8_t* wsl, int64_t* rowidx, float* ex) {
-  const int w = wave_id_uniform(), lane = lane_id(), nn = lane & 15, g = lane >> 4;
-  item_rows<MT>(a, first, len, rowidx);
-  __syncthreads();
-  int cols[2 * NB];
-#pragma unroll
-  for (int bb = 0; bb < NB; bb++) {
-    cols[2 * bb] = 128 * (c * NB + bb) + 16 * w;
-    cols[2 * bb + 1] = a.m + 128 * (c * NB + bb) + 16 * w;
-  }
-  f32x4 acc[MT][2 * NB];
-  gemm_item<MT, 2 * NB, MTMAX, 2>(a, e, cols, rowidx, abuf, sbuf, wsl, acc);
-  // epilogue per block and M-tile: gate/up tiles -> LDS [16][2][128] -> per row: H128, scale,
-  // SwiGLU, in_down, H128
-#pragma unroll
-  for (int bb = 0; bb < NB; bb++) {
-    const int cb = c * NB + bb;
-    const int64_t si = (int64_t)e * a.m + 128 * cb + 2 * lane;
-    const float og0 = f16_to_f32(a.out_gate[si]), og1 = f16_to_f32(a.out_gate[si + 1]);
-    const float ou0 = f16_to_f32(a.out_up[si]), ou1 = f16_to_f32(a.out_up[si + 1]);
-    const float id0 = f16_to_f32(a.in_down[si]), id1 = f16_to_f32(a.in_down[si + 1]);
-#pragma unroll
-    for (int mt = 0; mt < MT; mt++) {
-#pragma unroll
-      for (int i = 0; i < 4; i++) {
-        const int r = 4 * g + i;
-        ex[(r * 2 + 0) * 128 + 16 * w + nn] = acc[mt][2 * bb][i];
-        ex[(r * 2 + 1) * 128 + 16 * w + nn] = acc[mt][2 * bb + 1][i];
-      }
-      __syncthreads();
-#pragma unroll
-      for (int rr = 0; rr < 2; rr++) {
-        const int r = 2 * w + rr;  // 8 waves x 2 rows
-        const int pr = mt * 16 + r;
-        if (pr < len) {
-          float g0 = ex[(r * 2) * 128 + 2 * lane], g1 = ex[(r * 2) * 128 + 2 * lane + 1];
-          float u0 = ex[(r * 2 + 1) * 128 + 2 * lane], u1 = ex[(r * 2 + 1) * 128 + 2 * lane + 1];
+        for (int bb = 0; bb < 2; bb++) {
+          const float* row = ex + r * 512 + 128 * bb + 2 * lane;
+          float g0 = row[0], g1 = row[1], u0 = row[256], u1 = row[257];
           hadamard128_wave(g0, g1);
           hadamard128_wave(u0, u1);
-          float h0 = swiglu_bf16(g0 * og0, u0 * ou0) * id0;
-          float h1 = swiglu_bf16(g1 * og1, u1 * ou1) * id1;
+          float h0 = swiglu_bf16(g0 * og[bb][0], u0 * ou[bb][0]) * id[bb][0];
+          float h1 = swiglu_bf16(g1 * og[bb][1], u1 * ou[bb][1]) * id[bb][1];
           hadamard128_wave(h0, h1);
           uint32_t lo[kPfLo], sc[kPfLo];
           const uint32_t hi = hi_lo_terms(h0, h1, lo, sc);
-          const int64_t p = first + pr;
-          *reinterpret_cast<uint32_t*>(a.hhi + p * a.m + 128 * cb + 2 * lane) = hi;
+          const int64_t q = u.first + pr;
+          store_record(a.ha + (q * (a.m / 128) + c0 + bb) * kPfRecord, hi, lo);
 #pragma unroll
-          for (int t = 0; t < kPfLo; t++) {
-            *reinterpret_cast<uint16_t*>(a.hq + (t * a.nslots + p) * a.m + 128 * cb + 2 * lane) = (uint16_t)lo[t];
-            if (nn == 0) a.hs[(t * a.nslots + p) * (a.m / 32) + 4 * cb + g] = (uint8_t)sc[t];
-          }
+          for (int t = 0; t < kPfLo; t++)
+            if (nn == 0) a.hs[(t * a.nslots + q) * (a.m / 32) + 4 * (c0 + bb) + g] = (uint8_t)sc[t];
         }
       }
-      __syncthreads();
     }
+    __syncthreads();
   }
 }
-
-// ---------------------------------------------------------------- down GEMM + value finish
-// Item = (plan block b, output blocks ob NB .. ob NB + NB - 1 of 128); wave w owns tile 16w of each.
-template <int MT, int MTMAX, int NB>
-__device__ __forceinline__ void down_item(const PfGemm& a, int e, int first, int len, int ob, uint8_t* abuf, uint8_t* sbuf,
-                                          uint8_t* wsl, int64_t* rowidx, float* ex) {
+// down: a pass is the output columns [512 pass, +512); wave w owns tile w of each 128-block.
+template <int MT>
+__device__ __forceinline__ void down_finish(const PfGemm& a, const PfUnit& u, float* ex, const f32x4 (&acc)[MT][kPfTiles]) {
   const int w = wave_id_uniform(), lane = lane_id(), nn = lane & 15, g = lane >> 4;
-  item_rows<MT>(a, first, len, rowidx);
-  __syncthreads();
-  int cols[NB];
+  const int c0 = kPfCols * u.pass;
+  float od[4][2];
 #pragma unroll
-  for (int bb = 0; bb < NB; bb++) cols[bb] = 128 * (ob * NB + bb) + 16 * w;
-  f32x4 acc[MT][NB];
-  gemm_item<MT, NB, MTMAX, 2>(a, e, cols, rowidx, abuf, sbuf, wsl, acc);
+  for (int bb = 0; bb < 4; bb++)
 #pragma unroll
-  for (int bb = 0; bb < NB; bb++) {
-    const int cb = ob * NB + bb;
-    const int64_t si = (int64_t)e * a.N + 128 * cb + 2 * lane;
-    const float od0 = f16_to_f32(a.out_down[si]), od1 = f16_to_f32(a.out_down[si + 1]);
+    for (int i = 0; i < 2; i++) od[bb][i] = f16_to_f32(a.out_down[(int64_t)u.e * a.N + c0 + 128 * bb + 2 * lane + i]);
 #pragma unroll
-    for (int mt = 0; mt < MT; mt++) {
+  for (int mt = 0; mt < MT; mt++) {
 #pragma unroll
-      for (int i = 0; i < 4; i++) ex[(4 * g + i) * 128 + 16 * w + nn] = acc[mt][bb][i];
-      __syncthreads();
+    for (int j = 0; j < kPfTiles; j++)
 #pragma unroll
-      for (int rr = 0; rr < 2; rr++) {
-        const int r = 2 * w + rr;
-        const int pr = mt * 16 + r;
-        if (pr < len) {
-          float v0 = ex[r * 128 + 2 * lane], v1 = ex[r * 128 + 2 * lane + 1];
+      for (int i = 0; i < 4; i++) ex[(4 * g + i) * kPfCols + 128 * j + 16 * w + nn] = acc[mt][j][i];
+    __syncthreads();
+#pragma unroll
+    for (int rr = 0; rr < 2; rr++) {
+      const int r = 2 * w + rr;
+      const int pr = mt * 16 + r;
+      if (pr < u.len) {
+        const int slot = a.order[u.first + pr];
+#pragma unroll
+        for (int bb = 0; bb < 4; bb++) {
+          float v0 = ex[r * kPfCols + 128 * bb + 2 * lane], v1 = ex[r * kPfCols + 128 * bb + 2 * lane + 1];
           hadamard128_wave(v0, v1);
-          const int slot = a.order[first + pr];
-          const uint32_t pk = (uint32_t)f32_to_bf16(v0 * od0) | ((uint32_t)f32_to_bf16(v1 * od1) << 16);
-          *reinterpret_cast<uint32_t*>(a.values + (int64_t)slot * a.N + 128 * cb + 2 * lane) = pk;
+          const uint32_t pk = (uint32_t)f32_to_bf16(v0 * od[bb][0]) | ((uint32_t)f32_to_bf16(v1 * od[bb][1]) << 16);
+          *reinterpret_cast<uint32_t*>(a.values + (int64_t)slot * a.N + c0 + 128 * bb + 2 * lane) = pk;
         }
       }
-      __syncthreads();
     }
+    __syncthreads();
   }
 }
 
-// Grid: (plan blocks) x (output blocks per item).  Items of MTMIN..MTMAX M-tiles only (the others
-// exit at once).  Dynamic LDS: double-buffered activation stage, its scale stage and the row map
-// (the epilogue exchange reuses the stage), then per wave its tiles' weight scales.
-template <int MTMIN, int MTMAX>
-constexpr size_t pf_lds_bytes() {
-  return 2 * PfStage<MTMAX>::kBytes + 2 * PfStage<MTMAX>::kScaleBytes + MTMAX * 16 * sizeof(int64_t);
-}
-// per wave: NT tiles x 16 rows x K/32 scale bytes
-inline size_t pf_wscale_lds_bytes(int nt, int K) { return (size_t)kPfWaves * nt * 16 * (K / 32); }
-// 128-column output blocks per item: two for the small items (activations re-staged half as often
-// per weight byte), one for the large ones (register budget)
-__host__ __device__ constexpr int pf_blocks_per_item(int mtmax) { return mtmax <= 2 ? 2 : 1; }
-// LDS of the small and large GEMM kernels (GATE: gate/up, K = hidden; else down, K = intermediate)
-inline size_t pf_small_lds(bool gate, int K) {
-  return pf_lds_bytes<1, 2>() + pf_wscale_lds_bytes((gate ? 2 : 1) * pf_blocks_per_item(2), K);
-}
-inline size_t pf_large_lds(bool gate, int K) {
-  return pf_lds_bytes<3, 4>() + pf_wscale_lds_bytes((gate ? 2 : 1) * pf_blocks_per_item(4), K);
-}
-
-template <bool GATE, int MTMIN, int MTMAX>
-__device__ __forceinline__ void pf_gemm_body(const PfGemm& a, int bid) {
-  extern __shared__ __attribute__((aligned(16))) uint8_t pf_lds[];
-  uint8_t* abuf = pf_lds;
-  uint8_t* sbuf = abuf + 2 * PfStage<MTMAX>::kBytes;
-  int64_t* rowidx = reinterpret_cast<int64_t*>(sbuf + 2 * PfStage<MTMAX>::kScaleBytes);
-  static_assert(2 * PfStage<1>::kBytes >= 16 * 2 * 128 * 4, "the epilogue exchange must fit in the stage");
-  float* ex = reinterpret_cast<float*>(abuf);
-  constexpr int kNB = pf_blocks_per_item(MTMAX), kNT = GATE ? 2 * kNB : kNB;
-  uint8_t* wsl = pf_lds + pf_lds_bytes<MTMIN, MTMAX>() + wave_id_uniform() * kNT * 16 * (a.K / 32);
-  const int outblocks = (GATE ? a.m : a.N) / (128 * kNB);
-  // Workgroups are dealt to the 8 XCDs in turn.  Small items: the outblocks items of one plan block
-  // go to one XCD, so its activation rows are read into one L2 (workgroup i -> plan block
-  // 8 (i / 8 outblocks) + i % 8, output block (i % 8 outblocks) / 8).  Large items (the blocks of
-  // the popular experts): consecutive plan blocks of an output block share an XCD and its weights.
-  int b, ob;
-  if (MTMAX <= 2) {
-    const int grp = bid / (8 * outblocks), r = bid % (8 * outblocks);
-    b = 8 * grp + r % 8;
-    ob = r / 8;
-  } else {
-    b = bid / outblocks;
-    ob = bid % outblocks;
+// ---------------------------------------------------------------- the units of one class
+//   * Weights: a ring of kRing k steps in registers, through buffer loads: one offset register per
+//     lane, the tile and k step in the scalar offset (an expert's codes are below 4 GB).
+//   * Activations: stages of kSteps k steps, double buffered in LDS and shared by the waves; the
+//     next stage is in registers meanwhile and goes to LDS between this stage's MFMAs.
+//   * Weight scales: chunks of kScSteps k steps (16 rows per tile) in the wave's own LDS region.  (A
+//     byte load per lane and k step from memory costs about as much as the codes.)
+// When K / 128 is a multiple of kScSteps, all three run on from one unit into the next: the next unit
+// is claimed at the unit's start and its rows are looked up on the way, so that the last iteration's
+// loads are the next unit's first ones and are in flight during the finish.  Otherwise every unit
+// starts afresh.
+template <bool GATE, int MT>
+__device__ __forceinline__ void run_class(const PfGemm& a, int cls, uint8_t* lds) {
+  using S = PfShape<MT>;
+  constexpr int NT = kPfTiles, G = S::kSteps, D = S::kRing, B = S::kBurst, SC = S::kScSteps, kParts = SC / 2;  // 8 B parts per row
+  constexpr int U = D > 2 * G ? D : 2 * G;  // k steps per loop iteration: whole rings, both stage buffers
+  static_assert(D % B == 0 && U == D && U % (2 * G) == 0 && SC % U == 0 && SC >= 4 * U && U <= 4,
+                "ring, stage and scale chunk positions are fixed per step");
+  PfClass c;
+  c.queue = a.queue + cls * 8 * kPfQueueLine;
+  c.begin = cls ? a.ends[cls - 1] : 0;
+  c.n = a.ends[cls] - c.begin;
+  c.passes = pf_passes<GATE>(a);
+  if (c.n == 0) return;
+  float* ex = reinterpret_cast<float*>(lds);
+  uint8_t* abuf = lds + kPfExchange;
+  uint8_t* sbuf = abuf + 2 * S::kStageBytes;
+  int64_t* rowidx = reinterpret_cast<int64_t*>(sbuf + 2 * S::kAScales * 4);
+  int32_t* claimed = reinterpret_cast<int32_t*>(rowidx + S::kRows);
+  const int w = wave_id_uniform(), lane = lane_id(), nn = lane & 15, g = lane >> 4;
+  uint8_t* wsl = reinterpret_cast<uint8_t*>(claimed) + 16 + w * S::kScBytes;
+  const int xcd = (int)blockIdx.x % 8;
+  const int ksteps = a.K / 128, last = ksteps - 1;
+  const bool flow = ksteps % SC == 0;
+  // first weight row of column tile j in a pass
+  auto tile_row = [&](int pass, int j) {
+    return GATE ? (j & 1) * a.m + 256 * pass + 128 * (j >> 1) + 16 * w : kPfCols * pass + 128 * j + 16 * w;
+  };
+  const int sb = a.K / 32;  // scale bytes per weight row (a multiple of 8)
+  // what the loads read next: the current unit, in its last iteration the next one
+  __amdgpu_buffer_rsrc_t wres, sres;
+  int pass;
+  PfSrc<MT> src;
+  auto aim = [&](const PfUnit& u) {
+    wres = expert_rsrc(a.codes, u.e, (int64_t)a.N * (a.K / 2));
+    sres = expert_rsrc(a.wscales, u.e, (int64_t)a.N * sb);
+    pass = u.pass;
+    item_src<MT>(a, rowidx, src);
+  };
+  // lane (nn, g) holds row nn of its tile, k block g
+  const int woff = nn * (a.K / 2) + g * 16;
+  auto load_w = [&](i32x4 (&bw)[D][NT], int slot, int ks) {  // k steps ks .. ks + B - 1 into slot, slot + 1, ..
+#pragma unroll
+    for (int j = 0; j < NT; j++)
+#pragma unroll
+      for (int b = 0; b < B; b++)
+        bw[slot + b][j] =
+            __builtin_amdgcn_raw_buffer_load_b128(wres, woff, tile_row(pass, j) * (a.K / 2) + min(ks + b, last) * 64, 0);
+  };
+  // weight scales: 8 B part lane % kParts of row lane / kParts + i (64 / kParts)
+  constexpr int kScLoads = 16 * kParts / 64;
+  i32x2 scf[NT][kScLoads];
+  auto fetch_sc = [&](int ks) {  // parts past a row's end are its last part again
+    const int off = min(ks * 4 + (lane % kParts) * 8, sb - 8) + lane / kParts * sb;
+#pragma unroll
+    for (int j = 0; j < NT; j++)
+#pragma unroll
+      for (int i = 0; i < kScLoads; i++)
+        scf[j][i] = __builtin_amdgcn_raw_buffer_load_b64(sres, off, (tile_row(pass, j) + i * (64 / kParts)) * sb, 0);
+  };
+  auto put_sc = [&]() {
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int j = 0; j < NT; j++)
+#pragma unroll
+      for (int i = 0; i < kScLoads; i++)
+        *reinterpret_cast<i32x2*>(wsl + (j * 16 + lane / kParts + i * (64 / kParts)) * S::kScRow + lane % kParts * 8) = scf[j][i];
+    __builtin_amdgcn_wave_barrier();
+  };
+  const uint8_t* scrow = wsl + nn * S::kScRow + g;  // tile 0, first k step of the chunk
+  auto read_sc = [&](uint32_t (&bs)[NT], int ks) {
+#pragma unroll
+    for (int j = 0; j < NT; j++) bs[j] = scrow[j * 16 * S::kScRow + ks % SC * 4];
+  };
+  PfFetch<MT> f;
+  const PfLane at;
+  i32x4 bw[D][NT];
+  uint32_t bs[NT];
+  PfUnit cur{}, next{};
+  bool fresh = true;  // the unit's first loads are still to be issued
+  for (;;) {
+    if (fresh) {
+      __syncthreads();  // the LDS of the unit or class before is free
+      if (threadIdx.x == 0) *claimed = pf_settle(c, xcd, pf_claim(c, xcd));
+      __syncthreads();
+      const int v = __builtin_amdgcn_readfirstlane(*claimed);
+      if (v < 0) return;
+      cur = pf_unit(a, c, v);
+      unit_rows<MT>(a, cur, rowidx);
+      __syncthreads();
+      aim(cur);
+      fetch_sc(0);
+      fetch_k<MT>(src, 0, f);
+#pragma unroll
+      for (int d = 0; d < D; d += B) load_w(bw, d, d);
+      put_sc();
+      put_k<MT>(f, abuf, sbuf);
+      fetch_k<MT>(src, min(G, ksteps - G), f);
+      __syncthreads();
+      read_sc(bs, 0);
+    }
+    f32x4 acc[MT][NT];
+#pragma unroll
+    for (int mt = 0; mt < MT; mt++)
+#pragma unroll
+      for (int j = 0; j < NT; j++) acc[mt][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    int claim = 0;
+    bool more = false;
+    for (int ks = 0; ks < ksteps; ks += U) {
+      int back = 0;  // k step 0 of what the loads read, relative to this unit's end
+      if (flow) {    // block-uniform; the stage barriers order the steps
+        if (ks == 0 && threadIdx.x == 0) claim = pf_claim(c, xcd);
+        if (ks == U && threadIdx.x == 0) *claimed = pf_settle(c, xcd, claim);
+        if (ks == 2 * U) {
+          const int v = __builtin_amdgcn_readfirstlane(*claimed);
+          more = v >= 0;
+          next = cur;
+          if (more) next = pf_unit(a, c, v);
+          unit_rows<MT>(a, next, rowidx);
+        }
+        if (ks == ksteps - U) {
+          aim(next);
+          back = ksteps;
+        }
+      }
+      if ((ks + U) % SC == 0) fetch_sc(min(ks + U - back, last));
+#pragma unroll
+      for (int u = 0; u < U; u++) {
+        const int t = ks + u;  // block-uniform
+        if (U == 2 || t < ksteps) {  // K / 128 is even
+          constexpr int kBuf = S::kStageBytes, kSBuf = S::kAScales * 4;
+          const int now = (u / G) & 1;
+          const uint8_t* ab = abuf + now * kBuf + (u % G) * S::kStepBytes;
+          const uint8_t* asb = sbuf + now * kSBuf + (u % G) * S::kRows * kPfLo * 4;
+          PfLoRows lo;
+          u32x2 asc[MT];
+          gemm_hi<MT>(ab, asb, at, bw[u % D], bs, acc, lo, asc);
+          if (u % G == G - 1) {  // the next stage to LDS (past the end: not read), the one after to registers
+            put_k<MT>(f, abuf + (now ^ 1) * kBuf, sbuf + (now ^ 1) * kSBuf);
+            fetch_k<MT>(src, min(t + 1 + G - back, ksteps - G), f);
+          }
+          if (u == U - 1 && (ks + U) % SC == 0) put_sc();
+          uint32_t bsn[NT];
+          read_sc(bsn, t + 1);
+          gemm_lo<MT>(ab, at, bw[u % D], bs, acc, lo, asc);
+          if (u % B == B - 1) load_w(bw, u % D - (B - 1), t - (B - 1) + D - back);
+#pragma unroll
+          for (int j = 0; j < NT; j++) bs[j] = bsn[j];
+          if (u % G == G - 1) __syncthreads();
+        }
+      }
+    }
+    if (GATE)
+      gate_finish<MT>(a, cur, ex, acc);
+    else
+      down_finish<MT>(a, cur, ex, acc);
+    if (flow && !more) return;
+    cur = next;
+    fresh = !flow;
   }
-  if (b >= *a.nblk) return;
-  const int e = a.blk[b], first = a.blk[a.cap + b], len = a.blk[2 * a.cap + b];
-  const int mt = (len + 15) / 16;
-  if (mt < MTMIN || mt > MTMAX) return;
-#define PF_CASE(M)                                                                          \
-  case M:                                                                                   \
-    if (M >= MTMIN && M <= MTMAX) {                                                         \
-      if (GATE)                                                                             \
-        gateup_item<(M <= MTMAX ? M : 1), MTMAX, kNB>(a, e, first, len, ob, abuf, sbuf, wsl, rowidx, ex); \
-      else                                                                                  \
-        down_item<(M <= MTMAX ? M : 1), MTMAX, kNB>(a, e, first, len, ob, abuf, sbuf, wsl, rowidx, ex);     \
-    }                                                                                       \
-    break;
-  switch (mt) {
-    PF_CASE(1)
-    PF_CASE(2)
-    PF_CASE(3)
-    PF_CASE(4)
-    default: break;
-  }
-#undef PF_CASE
 }
 
-template <bool GATE, int MTMIN, int MTMAX>
-__global__ __launch_bounds__(kPfThreads) void pf_gemm_kernel(PfGemm a) {
-  pf_gemm_body<GATE, MTMIN, MTMAX>(a, (int)blockIdx.x);
-}
-
-// The down GEMM's small items (K = intermediate: 48 KB of LDS per block) held within 128 VGPRs so
-// that two blocks share a CU.
-__global__ __launch_bounds__(kPfThreads) __attribute__((amdgpu_waves_per_eu(4))) void pf_gemm_down_small_kernel(PfGemm a) {
-  pf_gemm_body<false, 1, 2>(a, (int)blockIdx.x);
-}
-
-// Both item classes in one launch: the large items' workgroups first (`nlarge` of them, a multiple
-// of 8 so that the small items keep their XCD mapping), so that the few long items of the popular
-// experts start at once and the many small ones fill the machine around them, instead of running
-// in a launch of their own after the small ones with most compute units idle.
+// One block per CU, every class in turn: a block that finds no unit of a class left goes on to the next.
 template <bool GATE>
-__global__ __launch_bounds__(kPfThreads) void pf_gemm_merged_kernel(PfGemm a, int nlarge) {
-  if ((int)blockIdx.x < nlarge)
-    pf_gemm_body<GATE, 3, 4>(a, (int)blockIdx.x);
-  else
-    pf_gemm_body<GATE, 1, 2>(a, (int)blockIdx.x - nlarge);
+__global__ __launch_bounds__(kPfThreads) __attribute__((amdgpu_waves_per_eu(2, 2))) void pf_gemm_kernel(PfGemm a) {
+  extern __shared__ __attribute__((aligned(16))) uint8_t pf_lds[];
+  run_class<GATE, 4>(a, 0, pf_lds);
+  run_class<GATE, 3>(a, 1, pf_lds);
+  run_class<GATE, 2>(a, 2, pf_lds);
+  run_class<GATE, 1>(a, 3, pf_lds);
 }
 
 template <bool GATE>
 int launch_pf_gemm(const PfGemm& a, hipStream_t s) {
-  const int n128 = (GATE ? a.m : a.N) / 128;  // 128-column output blocks
-  // whole groups of 8 plan blocks (b < *nblk <= cap is checked in the kernel)
-  const unsigned groups = (unsigned)((a.cap + 7) / 8 * 8);
-  const size_t small_lds = pf_small_lds(GATE, a.K), large_lds = pf_large_lds(GATE, a.K);
-  if (small_lds > kPfMaxLds || large_lds > kPfMaxLds)
-    return fail(MOE_EINVAL, "prefill GEMM needs %zu / %zu B of LDS (K = %d)", small_lds, large_lds, a.K);
   // dynamic LDS beyond 64 KB must be allowed explicitly (idempotent; cheap)
-  MOE_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&pf_gemm_kernel<GATE, 1, 2>),
-                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)small_lds));
-  MOE_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&pf_gemm_kernel<GATE, 3, 4>),
-                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)large_lds));
-  const unsigned nsmall = groups * (n128 / pf_blocks_per_item(2)), nlarge = groups * (n128 / pf_blocks_per_item(4));
-  if (GATE ? MOE_PF_MERGE_GATE : MOE_PF_MERGE_DOWN) {
-    const size_t lds = small_lds > large_lds ? small_lds : large_lds;
-    MOE_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&pf_gemm_merged_kernel<GATE>),
-                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-    hipLaunchKernelGGL((pf_gemm_merged_kernel<GATE>), dim3(nlarge + nsmall), dim3(kPfThreads), lds, s, a, (int)nlarge);
-    MOE_HIP(hipGetLastError());
-    return MOE_OK;
-  }
-  if (!GATE && MOE_PF_DOWN_TWO) {
-    MOE_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&pf_gemm_down_small_kernel),
-                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)small_lds));
-    hipLaunchKernelGGL(pf_gemm_down_small_kernel, dim3(nsmall), dim3(kPfThreads), small_lds, s, a);
-  } else {
-    hipLaunchKernelGGL((pf_gemm_kernel<GATE, 1, 2>), dim3(nsmall), dim3(kPfThreads), small_lds, s, a);
-  }
-  MOE_HIP(hipGetLastError());
-  hipLaunchKernelGGL((pf_gemm_kernel<GATE, 3, 4>), dim3(nlarge), dim3(kPfThreads), large_lds, s, a);
+  MOE_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&pf_gemm_kernel<GATE>),
+                              hipFuncAttributeMaxDynamicSharedMemorySize, kPfLds));
+  const int blocks = device_cus() > 0 ? device_cus() : 256;
+  hipLaunchKernelGGL((pf_gemm_kernel<GATE>), dim3((unsigned)blocks), dim3(kPfThreads), kPfLds, s, a);
   MOE_HIP(hipGetLastError());
   return MOE_OK;
 }
@@ -737,11 +893,12 @@ struct PfWorkspace {
   int32_t* starts;    // [E]
   int32_t* blk;       // [3][cap]
   int32_t* nblk;
-  uint16_t* xhi;      // [rows][h] fp16
-  uint8_t* xq;        // [kPfLo][rows][h] fp8 remainder terms
+  int32_t* ent;       // [cap]
+  int32_t* ends;      // [4]
+  int32_t* queue;     // [kPfQueueWords]
+  uint8_t* xa;        // [rows][h/128] records
   uint8_t* xs;        // [kPfLo][rows][h/32]
-  uint16_t* hhi;      // [n][m] fp16
-  uint8_t* hq;        // [kPfLo][n][m] fp8 remainder terms
+  uint8_t* ha;        // [n][m/128] records
   uint8_t* hs;        // [kPfLo][n][m/32]
   uint16_t* values;   // [n][h]
   int cap;
@@ -766,11 +923,12 @@ PfWorkspace pf_carve(void* base, int rows, int slots, int h, int m, int64_t expe
   w.starts = reinterpret_cast<int32_t*>(take((size_t)experts * 4));
   w.blk = reinterpret_cast<int32_t*>(take((size_t)3 * w.cap * 4));
   w.nblk = reinterpret_cast<int32_t*>(take(4));
-  w.xhi = reinterpret_cast<uint16_t*>(take((size_t)rows * h * 2));
-  w.xq = reinterpret_cast<uint8_t*>(take((size_t)kPfLo * rows * h));
+  w.ent = reinterpret_cast<int32_t*>(take((size_t)w.cap * 4));
+  w.ends = reinterpret_cast<int32_t*>(take(16));
+  w.queue = reinterpret_cast<int32_t*>(take(kPfQueueWords * 4));
+  w.xa = reinterpret_cast<uint8_t*>(take((size_t)rows * h * 4));
   w.xs = reinterpret_cast<uint8_t*>(take((size_t)kPfLo * rows * (h / 32)));
-  w.hhi = reinterpret_cast<uint16_t*>(take((size_t)n * m * 2));
-  w.hq = reinterpret_cast<uint8_t*>(take((size_t)kPfLo * n * m));
+  w.ha = reinterpret_cast<uint8_t*>(take((size_t)n * m * 4));
   w.hs = reinterpret_cast<uint8_t*>(take((size_t)kPfLo * n * (m / 32)));
   w.values = reinterpret_cast<uint16_t*>(take((size_t)n * h * 2));
   w.bytes = off;
@@ -858,9 +1016,8 @@ int mx_grouped_check(const uint16_t* x, const uint8_t* gate_up_codes, const uint
   MOE_ARG(hidden % 1024 == 0 && hidden > 0, "hidden must be a positive multiple of 1024 (got %d)", hidden);
   MOE_ARG(intermediate % 256 == 0 && intermediate > 0, "intermediate must be a positive multiple of 256 (got %d)",
           intermediate);
-  MOE_ARG(pf_small_lds(true, hidden) <= kPfMaxLds && pf_large_lds(true, hidden) <= kPfMaxLds &&
-              pf_small_lds(false, intermediate) <= kPfMaxLds && pf_large_lds(false, intermediate) <= kPfMaxLds,
-          "hidden %d / intermediate %d too large for the prefill GEMM's LDS", hidden, intermediate);
+  MOE_ARG(hidden <= kPfMaxHidden && intermediate <= kPfMaxIntermediate,
+          "hidden %d / intermediate %d too large for the prefill GEMM", hidden, intermediate);
   MOE_ARG(((uintptr_t)gate_up_scales | (uintptr_t)down_scales) % 16 == 0, "weight scale arrays must be 16-byte aligned");
   MOE_ARG(workspace != nullptr, "workspace must not be NULL");
   *w = pf_carve(const_cast<void*>(workspace), rows, slots, hidden, intermediate, experts);
@@ -884,8 +1041,8 @@ int mx_grouped_body(const uint16_t* x, int rows, int slots, const uint32_t* ids,
   if (rc) return rc;
   // activation terms
   const int64_t pwaves = (int64_t)rows * (hidden / 128);
-  hipLaunchKernelGGL(prep_terms_kernel, dim3((unsigned)((pwaves + 3) / 4)), dim3(256), 0, s, x, unit, rows, hidden,
-                     w.xhi, w.xq, w.xs);
+  hipLaunchKernelGGL(prep_terms_kernel, dim3((unsigned)((pwaves + 3) / 4) + 1), dim3(256), 0, s, x, unit, rows, hidden,
+                     w.xa, w.xs, w.blk, w.cap, w.nblk, w.ent, w.ends, w.queue);
   MOE_HIP(hipGetLastError());
   // gate/up GEMM + gate finish -> hidden terms
   PfGemm g{};
@@ -893,22 +1050,22 @@ int mx_grouped_body(const uint16_t* x, int rows, int slots, const uint32_t* ids,
   g.wscales = gate_up_scales;
   g.K = hidden;
   g.N = 2 * intermediate;
-  g.ahi = w.xhi;
-  g.aq = w.xq;
+  g.aa = w.xa;
   g.as = w.xs;
   g.arows = rows;
   g.rowmap = w.order;
   g.rowdiv = slots;
   g.blk = w.blk;
   g.cap = w.cap;
-  g.nblk = w.nblk;
+  g.ent = w.ent;
+  g.ends = w.ends;
+  g.queue = w.queue;
   g.order = w.order;
   g.out_gate = out_gate;
   g.out_up = out_up;
   g.in_down = in_down;
   g.m = intermediate;
-  g.hhi = w.hhi;
-  g.hq = w.hq;
+  g.ha = w.ha;
   g.hs = w.hs;
   g.nslots = n;
   if ((rc = launch_pf_gemm<true>(g, s))) return rc;
@@ -918,15 +1075,16 @@ int mx_grouped_body(const uint16_t* x, int rows, int slots, const uint32_t* ids,
   d.wscales = down_scales;
   d.K = intermediate;
   d.N = hidden;
-  d.ahi = w.hhi;
-  d.aq = w.hq;
+  d.aa = w.ha;
   d.as = w.hs;
   d.arows = n;
   d.rowmap = nullptr;
   d.rowdiv = 1;
   d.blk = w.blk;
   d.cap = w.cap;
-  d.nblk = w.nblk;
+  d.ent = w.ent;
+  d.ends = w.ends;
+  d.queue = w.queue + kPfQueueWords / 2;
   d.order = w.order;
   d.m = intermediate;
   d.out_down = out_down;
