@@ -15,14 +15,18 @@
 //     against the decoded fp16 weights (the codebook values are exact in fp16), so an M-tile of
 //     16 A rows carries 8 tokens.  The prep and gate-finish kernels write the A operand directly
 //     in the MFMA's k order (a_rh / a_j of the K4 tile rows), 256 B per row and 64-row quad.
-//   * A work item is (block of <= 64 sorted rows of one expert, 256 output columns; 128 for the
-//     last one when N % 256 == 128).  Each of the
-//     8 waves owns one set of 2 tiles (32 columns): per 64-row quad it loads its 16 B piece of the
-//     packed tiles, decodes it with the decode GEMV's piece decoder (LDS code table + arithmetic
-//     route) and runs 4 MFMAs per M-tile; the quad's A rows of the item are staged in LDS once
-//     for the 8 waves.  No split of K: every output is produced by one wave, no atomics.
-//   * Items are classed by M-tiles (1, 2, 4, 8) so small experts pay no padded MFMAs; each class
-//     is one persistent launch (the code table is loaded into LDS once per block).
+//   * A work item is (sorted rows of one expert, 256 output columns; 128 for the last one when
+//     N % 256 == 128).  Each of the 8 waves owns one set of 2 tiles (32 columns): per 64-row quad it
+//     loads its 16 B piece of the packed tiles, decodes it with the decode GEMV's piece decoder (LDS
+//     code table + arithmetic route) and runs 4 MFMAs per M-tile; the quad's A rows of the item are
+//     staged in LDS once for the 8 waves.  No split of K: every output is produced by one wave, no
+//     atomics.
+//   * Items are classed by M-tiles (1, 2, 4, for K4 also 8) so small experts pay no padded MFMAs; one
+//     persistent launch claims them largest first, two blocks per CU (80 KB of LDS each).
+//   * What bounds it: the decode's VALU work.  With 33..64 rows as two items of 32 rows (each decoding
+//     every piece) and A reads whose 16 rows shared four banks, the VALU was busy 84% and LDS 71% of
+//     the cycles; one item of 64 rows and conflict-free A lines: 76% and 47%, and the whole routed
+//     block of 1,501 rows (GLM-5.3 K4 layer) 4,721 -> 3,875 us, same outputs.
 //   * K2/K3 tiles (the K3 experts of the multi-token-prediction layer) take the same items and
 //     MFMAs; a lane reads the 4-5 words of the circular tile stream that hold its 32 codewords
 //     (the generic window of exlr8/metal/trellis.metal:25-40) and looks every codeword up in the
@@ -34,7 +38,9 @@
 #include "moe_device.h"
 #include "moe_host.h"
 
-// arithmetic pairs per even / odd word of the piece decoder (the rest read the code table)
+// arithmetic pairs per even / odd word of the piece decoder (the rest read the code table).  Whole routed
+// block of 1,501 / 300 / 40 rows: 2/2 3,844 / 1,818 / 1,111 us, 2/3 3,836 / 1,871 / 1,156, 1/2 3,925 /
+// 1,854 / 1,178, 1/1 4,009 / 1,970 / 1,278.
 #ifndef MOE_KP_ALU_EVEN
 #define MOE_KP_ALU_EVEN 2
 #endif
@@ -43,11 +49,8 @@
 #ifndef MOE_KP_PAIR
 #define MOE_KP_PAIR 2
 #endif
-#ifndef MOE_KP_MERGED
-#define MOE_KP_MERGED 1
-#endif
 #ifndef MOE_KP_ALU_ODD
-#define MOE_KP_ALU_ODD 3
+#define MOE_KP_ALU_ODD 2
 #endif
 
 namespace moe {
@@ -202,6 +205,11 @@ __device__ __forceinline__ void kp_generic_frags(const KpWords<KB>& p, int o, co
                       __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(q[2 * rh + 1][h], 1.0f, true));
 }
 
+// A rows in LDS: per M-tile (16 rows: hi and lo of 8 tokens) and row half 1 KB, k-group g's 16 B of row
+// m at 256 g + 16 (m ^ 2 g).  An MFMA operand read touches every 16 B column once per 16 lanes, and
+// eight neighbouring lanes of the staging writes hit eight columns: no bank conflicts in either.
+__device__ __forceinline__ int kp_a_slot(int m, int g) { return g * 256 + ((m ^ (2 * g)) * 16); }
+
 // One item: rows [first, first + len) of expert e (len <= 8 MT), projection proj, output columns
 // [256 cb, +256).  `ab` holds the two A stages (at least MT * 8 * kKpRowQuad bytes each), `tab` the
 // code table.  Every wave of the block runs it (it meets at block barriers).
@@ -214,7 +222,7 @@ __device__ __forceinline__ void kp_item(const KpGemm& a, const uint8_t* __restri
   const int nq = a.K / 64, it = a.K / 16, obs = a.N / 128;
   const int lane_off = (nn >> 3) * 128 + (nn & 7) * 16;
   const int src_lane = (lane & 7) == 0 ? lane + 7 : lane - 1;
-  const int s4 = w & 3;
+  const int s4 = w & 3, a_slot = kp_a_slot(nn, g);
   // K2/K3: the lane's first window bit b0 within its tile, and the tile words it reads
   constexpr int kNw = 8 * KB;
   const int b0 = (8 * 4 * (nn & 7) * KB + KB - 16 + 256 * KB) % (256 * KB), bo = b0 & 31;
@@ -260,7 +268,7 @@ __device__ __forceinline__ void kp_item(const KpGemm& a, const uint8_t* __restri
         const int row = c >> 4, part = c & 15;  // part = (rh * 2 + hl) * 4 + g
         const int rh = part >> 3, hl = (part >> 2) & 1, gg = part & 3;
         const int m = 2 * (row & 7) + hl;
-        *reinterpret_cast<i32x4*>(dst + (((row >> 3) * 2 + rh) * 16 + m) * 64 + gg * 16) = f[i];
+        *reinterpret_cast<i32x4*>(dst + ((row >> 3) * 2 + rh) * 1024 + kp_a_slot(m, gg)) = f[i];
       }
     }
   };
@@ -270,7 +278,7 @@ __device__ __forceinline__ void kp_item(const KpGemm& a, const uint8_t* __restri
   auto mfmas = [&](const uint8_t* ab, int rh, const f16x8& b0, const f16x8& b1) {
 #pragma unroll
     for (int mt = 0; mt < MT; mt++) {
-      const f16x8 av = *reinterpret_cast<const f16x8*>(ab + ((mt * 2 + rh) * 16 + nn) * 64 + g * 16);
+      const f16x8 av = *reinterpret_cast<const f16x8*>(ab + (mt * 2 + rh) * 1024 + a_slot);
       acc[mt][0] = __builtin_amdgcn_mfma_f32_16x16x32_f16(av, b0, acc[mt][0], 0, 0, 0);
       acc[mt][1] = __builtin_amdgcn_mfma_f32_16x16x32_f16(av, b1, acc[mt][1], 0, 0, 0);
     }
@@ -370,51 +378,112 @@ __device__ __forceinline__ void kp_item(const KpGemm& a, const uint8_t* __restri
       }
 }
 
-// MT M-tiles (8 rows each) per item: items of 8 (MT - 1) < len <= 8 MT rows (MT = 1, 2, 4, 8);
-// KB = trellis width
-template <int MT, int KB>
-__global__ __launch_bounds__(kKpThreads) void kp_gemm_kernel(KpGemm a) {
-  __shared__ __attribute__((aligned(16))) uint8_t tab[65536];
-  __shared__ __attribute__((aligned(16))) uint8_t abuf[2][MT * 8 * kKpRowQuad];
-  load_codebook_lds(tab, a.codebook);
+// A K4 item of 33..64 rows: every piece is decoded once for all of them (two items of 32 rows decode it
+// twice, and the decode is what bounds these launches).  The A rows are staged by row halves (32 of a
+// quad's 64 input rows), 8 KB per stage, so that the block stays at 80 KB of LDS and two share a CU.
+__device__ __forceinline__ void kp_item64(const KpGemm& a, const uint8_t* __restrict__ tab, uint8_t* ab0, uint8_t* ab1,
+                                          int e, int first, int len, int proj, int cb) {
+  constexpr int MT = 8;
+  const int w = wave_id_uniform(), lane = lane_id(), nn = lane & 15, g = lane >> 4;
+  const int nq = a.K / 64, it = a.K / 16, obs = a.N / 128;
+  const int src_lane = (lane & 7) == 0 ? lane + 7 : lane - 1;
+  const int s4 = w & 3, a_slot = kp_a_slot(nn, g);
+  const bool active = 2 * cb + (w >> 2) < obs;  // as in kp_item
+  const int ob = min(2 * cb + (w >> 2), obs - 1);
+  const uint8_t* wbase = a.packed[proj] + (nn >> 3) * 128 + (nn & 7) * 16 + 256 * s4;
+  auto piece = [&](int q) {
+    return *reinterpret_cast<const u32x4*>(wbase + chunk_offset(a.side, e, ob, 4 * q + g, it, obs));
+  };
+  // A staging: thread t brings 16 B part t % 8 ([hl][g]) of row t / 8
+  static_assert(kKpThreads == 8 * 64, "one chunk per thread and stage");
+  const int row = (int)threadIdx.x >> 3, part = (int)threadIdx.x & 7;
+  const uint8_t* asrc = reinterpret_cast<const uint8_t*>(a.a[proj]) + (int64_t)(first + min(row, len - 1)) * nq * kKpRowQuad + part * 16;
+  const int adst = (row >> 3) * 1024 + kp_a_slot(2 * (row & 7) + (part >> 2), part & 3);
+  f32x4 acc[MT][2];
+#pragma unroll
+  for (int mt = 0; mt < MT; mt++) acc[mt][0] = acc[mt][1] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  auto half = [&](const uint8_t* ab, uint32_t w0, uint32_t w1, uint32_t prior) {
+    if (!active) return;
+    f16x2 qv[2][4];
+    decode_pair_words_f16<MOE_KP_ALU_EVEN, MOE_KP_ALU_ODD>(w0, w1, prior, tab, qv);
+    const f16x8 b0 = frag(qv[0][0], qv[0][1], qv[1][0], qv[1][1]), b1 = frag(qv[0][2], qv[0][3], qv[1][2], qv[1][3]);
+    // each M-tile's A read is issued one M-tile ahead; the fences keep the eight reads (and the decode
+    // before them) from being live at once, which spills
+    __builtin_amdgcn_sched_barrier(0);
+    f16x8 av = *reinterpret_cast<const f16x8*>(ab + a_slot);
+#pragma unroll
+    for (int mt = 0; mt < MT; mt++) {
+      f16x8 next = av;
+      if (mt + 1 < MT) next = *reinterpret_cast<const f16x8*>(ab + (mt + 1) * 1024 + a_slot);
+      acc[mt][0] = __builtin_amdgcn_mfma_f32_16x16x32_f16(av, b0, acc[mt][0], 0, 0, 0);
+      acc[mt][1] = __builtin_amdgcn_mfma_f32_16x16x32_f16(av, b1, acc[mt][1], 0, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
+      av = next;
+    }
+    mfma_acc_guard(acc);
+  };
+  const int last = 2 * nq - 1;  // row halves
+  auto fetch_a = [&](int h) { return *reinterpret_cast<const i32x4*>(asrc + min(h, last) * 128); };
+  *reinterpret_cast<i32x4*>(ab0 + adst) = fetch_a(0);
+  u32x4 pc = piece(0);
+  i32x4 f = fetch_a(1);
   __syncthreads();
-  const int ncb = (a.N + kKpCols - 1) / kKpCols;
-  const int nblk = *a.nblk;
-  const int items = nblk * a.nproj * ncb;
-  for (int item = blockIdx.x; item < items; item += gridDim.x) {
-    const int cb = item % ncb, proj = (item / ncb) % a.nproj, b = item / (ncb * a.nproj);
-    const int len = a.blk[2 * a.cap + b];
-    if (len <= (MT / 2) * 8 || len > MT * 8) continue;  // another class
-    kp_item<MT, KB>(a, tab, abuf[0], abuf[1], a.blk[b], a.blk[a.cap + b], len, proj, cb);
+  for (int q = 0; q < nq; q++) {
+    const u32x4 pn = piece(min(q + 1, nq - 1));
+    const uint32_t prior = (uint32_t)__shfl((int)pc.w, src_lane, 64);
+    half(ab0, pc.x, pc.y, prior);
+    *reinterpret_cast<i32x4*>(ab1 + adst) = f;
+    f = fetch_a(2 * q + 2);
+    __syncthreads();
+    half(ab1, pc.z, pc.w, pc.y);
+    *reinterpret_cast<i32x4*>(ab0 + adst) = f;  // past the end: not read
+    f = fetch_a(2 * q + 3);
+    __syncthreads();
+    pc = pn;
   }
+#pragma unroll
+  for (int mt = 0; mt < MT; mt++)
+#pragma unroll
+    for (int h = 0; h < 2; h++)
+#pragma unroll
+      for (int tt = 0; tt < 2; tt++) {
+        const int r = mt * 8 + 2 * g + tt;
+        if (active && r < len) {
+          const int col = a.col_off[proj] + ob * 128 + 16 * (2 * s4 + (nn >> 3)) + (nn & 7) + 8 * h;
+          a.inner[(int64_t)(first + r) * a.inner_stride + col] =
+              fmaf(acc[mt][h][2 * tt + 1], 1.0f / 2048.0f, acc[mt][h][2 * tt]);
+        }
+      }
 }
 
-// The GEMMs' item entries, largest first: plan blocks of 17..64 rows as entries of up to 32 rows
-// (a block beyond 32 rows as two entries, its row halves: each row's sums are the same whatever
-// rows share its tiles), then blocks of 9..16 rows, then of up to 8.  One block of 256 threads
-// after the segment table; it also clears the two GEMMs' claim counters.
+// The GEMMs' item entries, largest first: plan blocks of 33..64 rows (whole, or with `halves` as two
+// entries, their row halves: each row's sums are the same whatever rows share its tiles), then blocks of
+// 17..32 rows, of 9..16, then of up to 8.  One block of 256 threads after the segment table; it also
+// clears the two GEMMs' claim counters.
 __global__ __launch_bounds__(256) void kp_order_kernel(const int32_t* __restrict__ blk, int cap,
                                                        const int32_t* __restrict__ nblk, int32_t* __restrict__ ent,
-                                                       int32_t* __restrict__ nent, int32_t* __restrict__ queue) {
-  __shared__ int32_t cnt[3], pos[3];
-  if (threadIdx.x < 3) cnt[threadIdx.x] = pos[threadIdx.x] = 0;
+                                                       int32_t* __restrict__ nent, int32_t* __restrict__ queue,
+                                                       int halves) {
+  __shared__ int32_t cnt[4], pos[4];
+  if (threadIdx.x < 4) cnt[threadIdx.x] = pos[threadIdx.x] = 0;
   __syncthreads();
   const int nb = min(*nblk, cap);
-  auto cls = [&](int len) { return len > 16 ? 0 : len > 8 ? 1 : 2; };
+  auto cls = [&](int len) { return len > 32 ? 0 : len > 16 ? 1 : len > 8 ? 2 : 3; };
+  auto entries = [&](int len) { return halves && len > 32 ? 2 : 1; };
   for (int b = threadIdx.x; b < nb; b += 256) {
     const int len = blk[2 * cap + b];
-    atomicAdd(&cnt[cls(len)], len > 32 ? 2 : 1);
+    atomicAdd(&cnt[cls(len)], entries(len));
   }
   __syncthreads();
   for (int b = threadIdx.x; b < nb; b += 256) {
     const int len = blk[2 * cap + b], c = cls(len);
-    const int base = (c > 0 ? cnt[0] : 0) + (c > 1 ? cnt[1] : 0);
-    const int at = base + atomicAdd(&pos[c], len > 32 ? 2 : 1);
+    const int base = (c > 0 ? cnt[0] : 0) + (c > 1 ? cnt[1] : 0) + (c > 2 ? cnt[2] : 0);
+    const int at = base + atomicAdd(&pos[c], entries(len));
     ent[at] = 2 * b;
-    if (len > 32) ent[at + 1] = 2 * b + 1;
+    if (entries(len) == 2) ent[at + 1] = 2 * b + 1;
   }
   if (threadIdx.x == 0) {
-    *nent = cnt[0] + cnt[1] + cnt[2];
+    *nent = cnt[0] + cnt[1] + cnt[2] + cnt[3];
     queue[0] = 0;
     queue[32] = 0;
   }
@@ -424,7 +493,7 @@ __global__ __launch_bounds__(256) void kp_order_kernel(const int32_t* __restrict
 // from a counter, so blocks that finish the long items go on to the short ones and the launch has
 // no class boundaries at which compute units wait for the last long item of a class.
 template <int KB>
-__global__ __launch_bounds__(kKpThreads) void kp_gemm_merged_kernel(KpGemm a) {
+__global__ __launch_bounds__(kKpThreads) __attribute__((amdgpu_waves_per_eu(4))) void kp_gemm_merged_kernel(KpGemm a) {
   __shared__ __attribute__((aligned(16))) uint8_t tab[65536];
   __shared__ __attribute__((aligned(16))) uint8_t abuf[2][4 * 8 * kKpRowQuad];
   // K2/K3 pieces hold more words: their registers allow one quad per step within 128 VGPRs
@@ -446,8 +515,11 @@ __global__ __launch_bounds__(kKpThreads) void kp_gemm_merged_kernel(KpGemm a) {
     const int b = en >> 1, half = en & 1;
     const int cb = r % ncb, proj = r / ncb;
     const int len = a.blk[2 * a.cap + b];
-    const int first = a.blk[a.cap + b] + 32 * half, n = half ? len - 32 : min(len, 32);
-    if (n > 16)
+    const int first = a.blk[a.cap + b] + 32 * half;
+    const int n = KB == 4 ? len : half ? len - 32 : min(len, 32);  // K4 blocks are whole
+    if (KB == 4 && n > 32)
+      kp_item64(a, tab, abuf[0], abuf[1], a.blk[b], first, n, proj, cb);
+    else if (n > 16)
       kp_item<4, KB>(a, tab, abuf[0], abuf[1], a.blk[b], first, n, proj, cb);
     else if (n > 8)
       kp_item<2, KB, kPair>(a, tab, abuf[0], abuf[0] + 2 * 8 * kKpRowQuad * kPair, a.blk[b], first, n, proj, cb);
@@ -584,22 +656,9 @@ KpWorkspace kp_carve(void* base, int64_t n, int h, int m, int64_t experts) {
 
 template <int KB>
 int launch_kp_gemm_k(const KpGemm& g, hipStream_t s) {
-  // persistent blocks, items strided over them.  The classes of up to 4 M-tiles fit two blocks per
-  // CU (68-80 KB of LDS) and get 4 blocks per CU queued, so the CUs stay busy to the end of the
-  // launch; the 8-tile class (96 KB) runs one block per CU.
+  // persistent blocks; two of them fit a CU (80 KB of LDS), and 4 per CU are queued
   const int blocks = device_cus() > 0 ? device_cus() : 256;
-  if (MOE_KP_MERGED) {
-    hipLaunchKernelGGL((kp_gemm_merged_kernel<KB>), dim3(4 * blocks), dim3(kKpThreads), 0, s, g);
-    MOE_HIP(hipGetLastError());
-    return MOE_OK;
-  }
-  hipLaunchKernelGGL((kp_gemm_kernel<1, KB>), dim3(4 * blocks), dim3(kKpThreads), 0, s, g);
-  MOE_HIP(hipGetLastError());
-  hipLaunchKernelGGL((kp_gemm_kernel<2, KB>), dim3(4 * blocks), dim3(kKpThreads), 0, s, g);
-  MOE_HIP(hipGetLastError());
-  hipLaunchKernelGGL((kp_gemm_kernel<4, KB>), dim3(4 * blocks), dim3(kKpThreads), 0, s, g);
-  MOE_HIP(hipGetLastError());
-  hipLaunchKernelGGL((kp_gemm_kernel<8, KB>), dim3(blocks), dim3(kKpThreads), 0, s, g);
+  hipLaunchKernelGGL((kp_gemm_merged_kernel<KB>), dim3(4 * blocks), dim3(kKpThreads), 0, s, g);
   MOE_HIP(hipGetLastError());
   return MOE_OK;
 }
@@ -653,7 +712,7 @@ int moe_trellis_grouped_mlp(int k, const uint16_t* x, const uint32_t* ids, int r
                                   (hipStream_t)stream)))
     return rc;
   hipLaunchKernelGGL(kp_order_kernel, dim3(1), dim3(256), 0, (hipStream_t)stream, w.blk, w.cap, w.nblk, w.ent, w.nent,
-                     w.queue);
+                     w.queue, k == 4 ? 0 : 1);
   MOE_HIP(hipGetLastError());
   const int64_t pw = kp_prep_waves(n, hidden, 2);
   hipLaunchKernelGGL(kp_prep_kernel, dim3((unsigned)((pw + 3) / 4)), dim3(256), 0, s, x, ids, w.order, w.counts, w.starts,
@@ -746,7 +805,7 @@ int moe_trellis_grouped_linear(int k, const uint16_t* x, int x_per_slot, const u
                                   (hipStream_t)stream)))
     return rc;
   hipLaunchKernelGGL(kp_order_kernel, dim3(1), dim3(256), 0, (hipStream_t)stream, w.blk, w.cap, w.nblk, w.ent, w.nent,
-                     w.queue);
+                     w.queue, k == 4 ? 0 : 1);
   MOE_HIP(hipGetLastError());
   const int64_t pw = kp_prep_waves(n, in_features, 1);
   hipLaunchKernelGGL(kp_prep_kernel, dim3((unsigned)((pw + 3) / 4)), dim3(256), 0, s, x, ids, w.order, w.counts, w.starts,
