@@ -58,22 +58,29 @@ __global__ __launch_bounds__(256) void router_logits_small(const uint16_t* __res
 }
 
 // ---------------------------------------------------------------- logits, prefill batches
-// 16 rows x 16 experts per block on the fp32 matrix cores (v_mfma_f32_16x16x4_f32); the 16 waves
-// split K into 16 chunks and the chunk tiles are summed in LDS in chunk order.  Which wave takes
-// which chunk rotates with the block, so the blocks do not all read the same k offsets at once.
-// Per 64-wide k step, lane l = 16 kk + r loads 16 consecutive k (32 B of x row r, 64 B of w row r)
-// at 16 kk: a row's four lanes read whole 128 B lines.  MFMA i (0..15) takes element i, so its
-// k-group kk covers k0 + 16 kk + i.
+// MR x NE tiles of 16 rows x 16 experts per block on the fp32 matrix cores
+// (v_mfma_f32_16x16x4_f32); the 16 waves split K into 16 chunks and the chunk tiles are summed in LDS
+// in chunk order, so a logit is the same bits whatever tile it is in.  Which wave takes which chunk
+// rotates with the block, so the blocks do not all read the same k offsets at once.  Per 64-wide k
+// step, lane l = 16 kk + r loads 16 consecutive k (32 B of x row r, 64 B of w row r) at 16 kk: a row's
+// four lanes read whole 128 B lines.  MFMA i (0..15) takes element i, so its k-group kk covers
+// k0 + 16 kk + i.
+// Bound by reads of x and w from L2: a 4 x 2 tile reads a third of what its logits cost as single tiles.
+// Hidden 6144, 256 experts, single tiles -> these: 1,024 rows 74 -> 43 us, 2,048 rows 143 -> 68 us (the
+// fp32 MFMAs alone need 41 us at 2,048).
 constexpr int kLogitWaves = 16;
+template <int MR, int NE>
 __global__ __launch_bounds__(kLogitWaves * 64) void router_logits_mfma(const uint16_t* __restrict__ x,
                                                                       const float* __restrict__ w, int rows,
                                                                       int hidden, int experts,
                                                                       float* __restrict__ logits) {
-  __shared__ f32x4 red[kLogitWaves][64];
+  extern __shared__ __attribute__((aligned(16))) uint8_t router_lds[];
+  f32x4* red = reinterpret_cast<f32x4*>(router_lds);  // [chunk][MR][NE][64]
+  constexpr int kTiles = MR * NE, kBatch = kTiles == 1 ? 2 : 1;  // 64-wide steps whose loads go out together
   // 1-D grid of (expert blocks) x (row blocks).  Workgroups are dealt to the 8 XCDs in turn; when
   // the expert blocks split evenly over them, XCD x takes expert blocks [x n/8, (x+1) n/8) for
   // every row block (its slice of w stays in its L2, and the row block's x is read once per XCD)
-  const int neb = (experts + 15) / 16;
+  const int neb = (experts + 16 * NE - 1) / (16 * NE);
   int bx, by;
   if (neb % 8 == 0) {
     const int per = neb / 8, j = blockIdx.x / 8;
@@ -83,46 +90,64 @@ __global__ __launch_bounds__(kLogitWaves * 64) void router_logits_mfma(const uin
     bx = blockIdx.x % neb;
     by = blockIdx.x / neb;
   }
-  const int r0 = by * 16, e0 = bx * 16;
+  const int r0 = by * 16 * MR, e0 = bx * 16 * NE;
   const int wv = wave_id_uniform(), lane = lane_id(), r = lane & 15, kk = lane >> 4;
   const int chunk = (wv + 5 * bx + 3 * by) % kLogitWaves;
   const int kq = hidden / kLogitWaves;  // a multiple of 64 (hidden % 1024 == 0)
-  const uint16_t* __restrict__ xr = x + (int64_t)min(r0 + r, rows - 1) * hidden + chunk * kq + 16 * kk;
-  const float* __restrict__ wr = w + (int64_t)min(e0 + r, experts - 1) * hidden + chunk * kq + 16 * kk;
-  f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
-  // two 64-wide steps per batch: all of a batch's loads are issued before its MFMAs
-  for (int k0 = 0; k0 < kq; k0 += 128) {
-    u32x4 xv[2][2];
-    f32x4 wvv[2][4];
+  const uint16_t* xr[MR];
+  const float* wr[NE];
 #pragma unroll
-    for (int b = 0; b < 2; b++) {
+  for (int i = 0; i < MR; i++) xr[i] = x + (int64_t)min(r0 + 16 * i + r, rows - 1) * hidden + chunk * kq + 16 * kk;
+#pragma unroll
+  for (int i = 0; i < NE; i++) wr[i] = w + (int64_t)min(e0 + 16 * i + r, experts - 1) * hidden + chunk * kq + 16 * kk;
+  f32x4 acc[MR][NE];
+#pragma unroll
+  for (int m = 0; m < MR; m++)
+#pragma unroll
+    for (int n = 0; n < NE; n++) acc[m][n] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  for (int k0 = 0; k0 < kq; k0 += 64 * kBatch) {
+    u32x4 xv[kBatch][MR][2];
+    f32x4 wvv[kBatch][NE][4];
+#pragma unroll
+    for (int b = 0; b < kBatch; b++) {
       const int k = min(k0 + 64 * b, kq - 64);  // past the end: re-read the last step (not used)
 #pragma unroll
-      for (int i = 0; i < 2; i++) xv[b][i] = *reinterpret_cast<const u32x4*>(xr + k + 8 * i);
+      for (int m = 0; m < MR; m++)
 #pragma unroll
-      for (int i = 0; i < 4; i++) wvv[b][i] = *reinterpret_cast<const f32x4*>(wr + k + 4 * i);
+        for (int i = 0; i < 2; i++) xv[b][m][i] = *reinterpret_cast<const u32x4*>(xr[m] + k + 8 * i);
+#pragma unroll
+      for (int n = 0; n < NE; n++)
+#pragma unroll
+        for (int i = 0; i < 4; i++) wvv[b][n][i] = *reinterpret_cast<const f32x4*>(wr[n] + k + 4 * i);
     }
 #pragma unroll
-    for (int b = 0; b < 2; b++) {
+    for (int b = 0; b < kBatch; b++) {
       if (k0 + 64 * b < kq) {
 #pragma unroll
-        for (int i = 0; i < 16; i++) {
-          const uint32_t xw = xv[b][i >> 3][(i >> 1) & 3];
-          const float xa = bf16_to_f32((uint16_t)((i & 1) ? (xw >> 16) : (xw & 0xFFFFu)));
-          acc = __builtin_amdgcn_mfma_f32_16x16x4f32(xa, wvv[b][i >> 2][i & 3], acc, 0, 0, 0);
-        }
+        for (int i = 0; i < 16; i++)
+#pragma unroll
+          for (int m = 0; m < MR; m++) {
+            const uint32_t xw = xv[b][m][i >> 3][(i >> 1) & 3];
+            const float xa = bf16_to_f32((uint16_t)((i & 1) ? (xw >> 16) : (xw & 0xFFFFu)));
+#pragma unroll
+            for (int n = 0; n < NE; n++)
+              acc[m][n] = __builtin_amdgcn_mfma_f32_16x16x4f32(xa, wvv[b][n][i >> 2][i & 3], acc[m][n], 0, 0, 0);
+          }
       }
     }
   }
-  red[chunk][lane] = acc;
-  __syncthreads();
-  if (wv == 0) {
-    f32x4 t = red[0][lane];
 #pragma unroll
-    for (int i = 1; i < kLogitWaves; i++) t = t + red[i][lane];
+  for (int m = 0; m < MR; m++)
+#pragma unroll
+    for (int n = 0; n < NE; n++) red[(chunk * kTiles + m * NE + n) * 64 + lane] = acc[m][n];
+  __syncthreads();
+  if (wv < kTiles) {
+    f32x4 t = red[wv * 64 + lane];
+#pragma unroll
+    for (int i = 1; i < kLogitWaves; i++) t = t + red[(i * kTiles + wv) * 64 + lane];
 #pragma unroll
     for (int i = 0; i < 4; i++) {
-      const int row = r0 + 4 * kk + i, e = e0 + r;  // D[4 kk + i][r]
+      const int row = r0 + 16 * (wv / NE) + 4 * kk + i, e = e0 + 16 * (wv % NE) + r;  // D[4 kk + i][r]
       if (row < rows && e < experts) logits[(int64_t)row * experts + e] = t[i];
     }
   }
@@ -312,9 +337,26 @@ int launch_router_logits(const uint16_t* x, const float* w, int rows, int hidden
     hipLaunchKernelGGL(router_logits_small<kMaxRows>, dim3(experts), dim3(256), 0, s, x, w, rows, hidden, experts,
                        logits);
   } else {
-    const unsigned grid = (unsigned)((experts + 15) / 16) * (unsigned)((rows + 15) / 16);
-    hipLaunchKernelGGL(router_logits_mfma, dim3(grid), dim3(kLogitWaves * 64), 0, s, x, w, rows, hidden, experts,
-                       logits);
+    // the smallest tile whose blocks fit the CUs at once (single tiles: two blocks per CU): a launch takes
+    // as long as a CU's blocks, 40 us of two single tiles, 43 of one 2 x 2, 68 of one 4 x 2
+    const int cus = device_cus() > 0 ? device_cus() : 256;
+    auto blocks = [&](int mr, int ne) { return (int64_t)((experts + 16 * ne - 1) / (16 * ne)) * ((rows + 16 * mr - 1) / (16 * mr)); };
+    int rc = MOE_OK;
+    auto launch = [&](auto kernel, int mr, int ne) {
+      const int lds = kLogitWaves * mr * ne * 1024;
+      if (hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, lds) != hipSuccess)
+        rc = fail(MOE_ENOTSUP, "router logits need %d B of LDS", lds);
+      else
+        hipLaunchKernelGGL(kernel, dim3((unsigned)blocks(mr, ne)), dim3(kLogitWaves * 64), lds, s, x, w, rows, hidden,
+                           experts, logits);
+    };
+    if (blocks(1, 1) <= 2 * cus)
+      launch(&router_logits_mfma<1, 1>, 1, 1);
+    else if (blocks(2, 2) <= cus)
+      launch(&router_logits_mfma<2, 2>, 2, 2);
+    else
+      launch(&router_logits_mfma<4, 2>, 4, 2);
+    if (rc) return rc;
   }
   MOE_HIP(hipGetLastError());
   return MOE_OK;
