@@ -21,12 +21,13 @@
 //     code table + arithmetic route) and runs 4 MFMAs per M-tile; the quad's A rows of the item are
 //     staged in LDS once for the 8 waves.  No split of K: every output is produced by one wave, no
 //     atomics.
-//   * Items are classed by M-tiles (1, 2, 4, for K4 also 8) so small experts pay no padded MFMAs; one
+//   * Items are classed by M-tiles (1, 2, 4, for K4 and K3 also 8) so small experts pay no padded MFMAs; one
 //     persistent launch claims them largest first, two blocks per CU (80 KB of LDS each).
 //   * What bounds it: the decode's VALU work.  With 33..64 rows as two items of 32 rows (each decoding
 //     every piece) and A reads whose 16 rows shared four banks, the VALU was busy 84% and LDS 71% of
 //     the cycles; one item of 64 rows and conflict-free A lines: 76% and 47%, and the whole routed
 //     block of 1,501 rows (GLM-5.3 K4 layer) 4,721 -> 3,875 us, same outputs.
+//     K3 layer, 300 / 800 rows: 2,560 / 3,562 -> 2,444 / 3,132 us.
 //   * K2/K3 tiles (the K3 experts of the multi-token-prediction layer) take the same items and
 //     MFMAs; a lane reads the 4-5 words of the circular tile stream that hold its 32 codewords
 //     (the generic window of exlr8/metal/trellis.metal:25-40) and looks every codeword up in the
@@ -171,24 +172,24 @@ struct KpWords {
   uint32_t v[kStream + 1];                                   // from word b0 / 32 on (circular)
 };
 
-// The lane's two B fragments per row half rh (h = 0: slots 0-3, h = 1: slots 4-7 of each tile
-// lane), in the order the K4 piece decoder gives them; o = b0 % 32.
+// The lane's two B fragments of row half rh (h = 0: slots 0-3, h = 1: slots 4-7 of the tile lanes
+// L0 + 2 rh, L0 + 2 rh + 1), in the order the K4 piece decoder gives them; o = b0 % 32.
 template <int KB>
-__device__ __forceinline__ void kp_generic_frags(const KpWords<KB>& p, int o, const uint8_t* __restrict__ tab,
-                                                 f16x8 (&b)[2][2]) {
+__device__ __forceinline__ void kp_generic_half(const KpWords<KB>& p, int o, const uint8_t* __restrict__ tab, int rh,
+                                                f16x8 (&b)[2]) {
   constexpr int S = KpWords<KB>::kStream;
   uint32_t u[S];  // the stream from bit b0 on
 #pragma unroll
   for (int k = 0; k < S; k++) u[k] = (uint32_t)(((((uint64_t)p.v[k]) << 32 | p.v[k + 1]) << o) >> 32);
-  uint32_t q[4][2];  // [tile lane L0 + i][h]: the E4M3 bytes of 4 codewords
+  uint32_t q[2][2];  // [tile lane L0 + 2 rh + i][h]: the E4M3 bytes of 4 codewords
 #pragma unroll
-  for (int i = 0; i < 4; i++)
+  for (int i = 0; i < 2; i++)
 #pragma unroll
     for (int h = 0; h < 2; h++) {
       uint32_t pk = 0;
 #pragma unroll
       for (int t = 0; t < 4; t++) {
-        const int pos = (8 * i + 4 * h + t) * KB, wi = pos / 32, off = pos % 32;
+        const int pos = (8 * (2 * rh + i) + 4 * h + t) * KB, wi = pos / 32, off = pos % 32;
         const uint32_t cw = off <= 16 ? (u[wi] >> (16 - off)) & 0xFFFFu
                                       : __builtin_amdgcn_alignbit(u[wi], u[min(wi + 1, S - 1)], 48 - off) & 0xFFFFu;
         pk |= (uint32_t)tab[cw] << (8 * t);
@@ -196,13 +197,17 @@ __device__ __forceinline__ void kp_generic_frags(const KpWords<KB>& p, int o, co
       q[i][h] = pk;
     }
 #pragma unroll
-  for (int rh = 0; rh < 2; rh++)
-#pragma unroll
-    for (int h = 0; h < 2; h++)
-      b[rh][h] = frag(__builtin_amdgcn_cvt_scalef32_pk_f16_fp8(q[2 * rh][h], 1.0f, false),
-                      __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(q[2 * rh][h], 1.0f, true),
-                      __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(q[2 * rh + 1][h], 1.0f, false),
-                      __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(q[2 * rh + 1][h], 1.0f, true));
+  for (int h = 0; h < 2; h++)
+    b[h] = frag(__builtin_amdgcn_cvt_scalef32_pk_f16_fp8(q[0][h], 1.0f, false),
+                __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(q[0][h], 1.0f, true),
+                __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(q[1][h], 1.0f, false),
+                __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(q[1][h], 1.0f, true));
+}
+template <int KB>
+__device__ __forceinline__ void kp_generic_frags(const KpWords<KB>& p, int o, const uint8_t* __restrict__ tab,
+                                                 f16x8 (&b)[2][2]) {
+  kp_generic_half<KB>(p, o, tab, 0, b[0]);
+  kp_generic_half<KB>(p, o, tab, 1, b[1]);
 }
 
 // A rows in LDS: per M-tile (16 rows: hi and lo of 8 tokens) and row half 1 KB, k-group g's 16 B of row
@@ -378,9 +383,10 @@ __device__ __forceinline__ void kp_item(const KpGemm& a, const uint8_t* __restri
       }
 }
 
-// A K4 item of 33..64 rows: every piece is decoded once for all of them (two items of 32 rows decode it
+// A K4 or K3 item of 33..64 rows: every piece is decoded once for all of them (two items of 32 rows decode it
 // twice, and the decode is what bounds these launches).  The A rows are staged by row halves (32 of a
 // quad's 64 input rows), 8 KB per stage, so that the block stays at 80 KB of LDS and two share a CU.
+template <int KB>
 __device__ __forceinline__ void kp_item64(const KpGemm& a, const uint8_t* __restrict__ tab, uint8_t* ab0, uint8_t* ab1,
                                           int e, int first, int len, int proj, int cb) {
   constexpr int MT = 8;
@@ -390,9 +396,23 @@ __device__ __forceinline__ void kp_item64(const KpGemm& a, const uint8_t* __rest
   const int s4 = w & 3, a_slot = kp_a_slot(nn, g);
   const bool active = 2 * cb + (w >> 2) < obs;  // as in kp_item
   const int ob = min(2 * cb + (w >> 2), obs - 1);
-  const uint8_t* wbase = a.packed[proj] + (nn >> 3) * 128 + (nn & 7) * 16 + 256 * s4;
-  auto piece = [&](int q) {
-    return *reinterpret_cast<const u32x4*>(wbase + chunk_offset(a.side, e, ob, 4 * q + g, it, obs));
+  // the lane's pieces, as in kp_item
+  constexpr int kNw = 8 * KB;
+  const int b0 = (8 * 4 * (nn & 7) * KB + KB - 16 + 256 * KB) % (256 * KB), bo = b0 & 31;
+  using Piece = std::conditional_t<KB == 4, u32x4, KpWords<KB>>;
+  const uint8_t* wbase =
+      a.packed[proj] + (KB == 4 ? (nn >> 3) * 128 + (nn & 7) * 16 + 256 * s4 : 32 * KB * (2 * s4 + (nn >> 3)));
+  auto piece = [&](int q) -> Piece {
+    if constexpr (KB == 4) {
+      return *reinterpret_cast<const u32x4*>(wbase + chunk_offset(a.side, e, ob, 4 * q + g, it, obs));
+    } else {
+      const uint32_t* t =
+          reinterpret_cast<const uint32_t*>(wbase + chunk_index(a.side, e, ob, 4 * q + g, it, obs) * (256 * KB));
+      Piece r;
+#pragma unroll
+      for (int k = 0; k <= KpWords<KB>::kStream; k++) r.v[k] = t[(b0 / 32 + k) % kNw];
+      return r;
+    }
   };
   // A staging: thread t brings 16 B part t % 8 ([hl][g]) of row t / 8
   static_assert(kKpThreads == 8 * 64, "one chunk per thread and stage");
@@ -402,11 +422,20 @@ __device__ __forceinline__ void kp_item64(const KpGemm& a, const uint8_t* __rest
   f32x4 acc[MT][2];
 #pragma unroll
   for (int mt = 0; mt < MT; mt++) acc[mt][0] = acc[mt][1] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-  auto half = [&](const uint8_t* ab, uint32_t w0, uint32_t w1, uint32_t prior) {
+  auto half = [&](const uint8_t* ab, const Piece& pc, int rh) {
     if (!active) return;
-    f16x2 qv[2][4];
-    decode_pair_words_f16<MOE_KP_ALU_EVEN, MOE_KP_ALU_ODD>(w0, w1, prior, tab, qv);
-    const f16x8 b0 = frag(qv[0][0], qv[0][1], qv[1][0], qv[1][1]), b1 = frag(qv[0][2], qv[0][3], qv[1][2], qv[1][3]);
+    f16x8 b[2];
+    if constexpr (KB == 4) {
+      f16x2 qv[2][4];
+      if (rh == 0)
+        decode_pair_words_f16<MOE_KP_ALU_EVEN, MOE_KP_ALU_ODD>(pc.x, pc.y, (uint32_t)__shfl((int)pc.w, src_lane, 64), tab, qv);
+      else
+        decode_pair_words_f16<MOE_KP_ALU_EVEN, MOE_KP_ALU_ODD>(pc.z, pc.w, pc.y, tab, qv);
+      b[0] = frag(qv[0][0], qv[0][1], qv[1][0], qv[1][1]);
+      b[1] = frag(qv[0][2], qv[0][3], qv[1][2], qv[1][3]);
+    } else {
+      kp_generic_half<KB>(pc, bo, tab, rh, b);
+    }
     // each M-tile's A read is issued one M-tile ahead; the fences keep the eight reads (and the decode
     // before them) from being live at once, which spills
     __builtin_amdgcn_sched_barrier(0);
@@ -415,8 +444,8 @@ __device__ __forceinline__ void kp_item64(const KpGemm& a, const uint8_t* __rest
     for (int mt = 0; mt < MT; mt++) {
       f16x8 next = av;
       if (mt + 1 < MT) next = *reinterpret_cast<const f16x8*>(ab + (mt + 1) * 1024 + a_slot);
-      acc[mt][0] = __builtin_amdgcn_mfma_f32_16x16x32_f16(av, b0, acc[mt][0], 0, 0, 0);
-      acc[mt][1] = __builtin_amdgcn_mfma_f32_16x16x32_f16(av, b1, acc[mt][1], 0, 0, 0);
+      acc[mt][0] = __builtin_amdgcn_mfma_f32_16x16x32_f16(av, b[0], acc[mt][0], 0, 0, 0);
+      acc[mt][1] = __builtin_amdgcn_mfma_f32_16x16x32_f16(av, b[1], acc[mt][1], 0, 0, 0);
       __builtin_amdgcn_sched_barrier(0);
       av = next;
     }
@@ -425,17 +454,16 @@ __device__ __forceinline__ void kp_item64(const KpGemm& a, const uint8_t* __rest
   const int last = 2 * nq - 1;  // row halves
   auto fetch_a = [&](int h) { return *reinterpret_cast<const i32x4*>(asrc + min(h, last) * 128); };
   *reinterpret_cast<i32x4*>(ab0 + adst) = fetch_a(0);
-  u32x4 pc = piece(0);
+  Piece pc = piece(0);
   i32x4 f = fetch_a(1);
   __syncthreads();
   for (int q = 0; q < nq; q++) {
-    const u32x4 pn = piece(min(q + 1, nq - 1));
-    const uint32_t prior = (uint32_t)__shfl((int)pc.w, src_lane, 64);
-    half(ab0, pc.x, pc.y, prior);
+    const Piece pn = piece(min(q + 1, nq - 1));
+    half(ab0, pc, 0);
     *reinterpret_cast<i32x4*>(ab1 + adst) = f;
     f = fetch_a(2 * q + 2);
     __syncthreads();
-    half(ab1, pc.z, pc.w, pc.y);
+    half(ab1, pc, 1);
     *reinterpret_cast<i32x4*>(ab0 + adst) = f;  // past the end: not read
     f = fetch_a(2 * q + 3);
     __syncthreads();
@@ -516,9 +544,9 @@ __global__ __launch_bounds__(kKpThreads) __attribute__((amdgpu_waves_per_eu(4)))
     const int cb = r % ncb, proj = r / ncb;
     const int len = a.blk[2 * a.cap + b];
     const int first = a.blk[a.cap + b] + 32 * half;
-    const int n = KB == 4 ? len : half ? len - 32 : min(len, 32);  // K4 blocks are whole
-    if (KB == 4 && n > 32)
-      kp_item64(a, tab, abuf[0], abuf[1], a.blk[b], first, n, proj, cb);
+    const int n = KB >= 3 ? len : half ? len - 32 : min(len, 32);  // K4 and K3 blocks are whole
+    if (KB >= 3 && n > 32)
+      kp_item64<(KB >= 3 ? KB : 4)>(a, tab, abuf[0], abuf[1], a.blk[b], first, n, proj, cb);
     else if (n > 16)
       kp_item<4, KB>(a, tab, abuf[0], abuf[1], a.blk[b], first, n, proj, cb);
     else if (n > 8)
@@ -712,7 +740,7 @@ int moe_trellis_grouped_mlp(int k, const uint16_t* x, const uint32_t* ids, int r
                                   (hipStream_t)stream)))
     return rc;
   hipLaunchKernelGGL(kp_order_kernel, dim3(1), dim3(256), 0, (hipStream_t)stream, w.blk, w.cap, w.nblk, w.ent, w.nent,
-                     w.queue, k == 4 ? 0 : 1);
+                     w.queue, k >= 3 ? 0 : 1);
   MOE_HIP(hipGetLastError());
   const int64_t pw = kp_prep_waves(n, hidden, 2);
   hipLaunchKernelGGL(kp_prep_kernel, dim3((unsigned)((pw + 3) / 4)), dim3(256), 0, s, x, ids, w.order, w.counts, w.starts,
@@ -805,7 +833,7 @@ int moe_trellis_grouped_linear(int k, const uint16_t* x, int x_per_slot, const u
                                   (hipStream_t)stream)))
     return rc;
   hipLaunchKernelGGL(kp_order_kernel, dim3(1), dim3(256), 0, (hipStream_t)stream, w.blk, w.cap, w.nblk, w.ent, w.nent,
-                     w.queue, k == 4 ? 0 : 1);
+                     w.queue, k >= 3 ? 0 : 1);
   MOE_HIP(hipGetLastError());
   const int64_t pw = kp_prep_waves(n, in_features, 1);
   hipLaunchKernelGGL(kp_prep_kernel, dim3((unsigned)((pw + 3) / 4)), dim3(256), 0, s, x, ids, w.order, w.counts, w.starts,
